@@ -32,6 +32,7 @@
 #include "nh_ocv.h"
 #include "nh_internal.h"
 #include "nh_pool.h"
+#include "nh_xfer.h"
 
 using namespace onh;
 
@@ -274,6 +275,7 @@ void release(orctm_nh_t* h) {
   free_all(h);
   if (h->stream) hipStreamDestroy(h->stream);
   delete h;
+  xfer_release();
 }
 
 // Tiles (64 x h columns) of one system in natural (row-major) order.
@@ -1272,6 +1274,7 @@ int orctm_nh_create(const orctm_nh_grid_t* grid, const orctm_nh_options_t* opts,
   if (strncmp(prop.gcnArchName, "gfx950", 6) != 0) return ORCTM_NH_ERR_NODEVICE;
   orctm_nh_t* h = new (std::nothrow) orctm_nh_t();
   if (!h) return ORCTM_NH_ERR_NOMEM;
+  xfer_retain();
   h->opts = o;
   h->op = std::make_shared<OpData>();
   h->op->device = o.device;
@@ -1320,7 +1323,8 @@ int orctm_nh_set_rhs(orctm_nh_t* h, const double* divg) {
   const int rc = ensure_ctx(h);
   if (rc != ORCTM_NH_OK) return rc;
   hipError_t e = ensure_fort(h);
-  if (e == hipSuccess) e = hipMemcpyAsync(h->d_fort, divg, n * sizeof(double), hipMemcpyHostToDevice, h->stream);
+  const XferPiece in = xfer_flat(h->d_fort, divg, n * sizeof(double));
+  if (e == hipSuccess) e = xfer_to_device(h->opts.device, h->stream, &in, 1);
   if (e == hipSuccess)
     e = launch_rhs(h->stream, h->ctx.d_sys, h->ctx.d_tiles, h->ctx.ntiles, 1, h->d_fort, h->IE, h->JE);
   if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
@@ -1336,7 +1340,8 @@ int orctm_nh_set_guess(orctm_nh_t* h, const double* pnh) {
   const int rc = ensure_ctx(h);
   if (rc != ORCTM_NH_OK) return rc;
   hipError_t e = ensure_fort(h);
-  if (e == hipSuccess) e = hipMemcpyAsync(h->d_fort, pnh, n * sizeof(double), hipMemcpyHostToDevice, h->stream);
+  const XferPiece in = xfer_flat(h->d_fort, pnh, n * sizeof(double));
+  if (e == hipSuccess) e = xfer_to_device(h->opts.device, h->stream, &in, 1);
   if (e == hipSuccess)
     e = launch_guess(h->stream, h->ctx.d_sys, h->ctx.d_tiles, h->ctx.ntiles, h->d_fort, h->IE, h->JE);
   if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
@@ -1365,14 +1370,8 @@ int orctm_nh_get_solution(orctm_nh_t* h, double* pnh) {
   DEVLOCK;
   hipSetDevice(h->opts.device);
   // interior only (mo_petsc.f90:223-227); the halo of pnh is left as it is
-  for (int k = 0; k < h->nz; ++k) {
-    double* dst = pnh + 1 + (size_t)h->IE * (1 + (size_t)h->JE * k);
-    const double* src = h->sys.p64 + (size_t)k * h->plane;
-    hipError_t e = hipMemcpy2D(dst, (size_t)h->IE * 8, src, (size_t)h->pitch * 8, (size_t)h->nx * 8, (size_t)h->ny,
-                               hipMemcpyDeviceToHost);
-    if (e != hipSuccess) return map_err(e);
-  }
-  return ORCTM_NH_OK;
+  const XferPiece out = xfer_interior(h->sys.p64, pnh, h->IE, h->JE, h->KE, h->pitch, h->plane);
+  return map_err(xfer_to_host(h->opts.device, h->stream, &out, 1));
 }
 
 int orctm_nh_solve(orctm_nh_t* h, const double* divg, double* pnh, orctm_nh_stats_t* st) {
@@ -1570,6 +1569,7 @@ int orctm_nh_clone(orctm_nh_t* src, orctm_nh_t** out) {
   hipSetDevice(src->opts.device);
   orctm_nh_t* h = new (std::nothrow) orctm_nh_t();
   if (!h) return ORCTM_NH_ERR_NOMEM;
+  xfer_retain();
   h->opts = src->opts;
   h->op = src->op;
   h->IE = src->IE;
@@ -1741,13 +1741,11 @@ int orctm_nh_divergence(orctm_nh_t* h, const double* uoo, const double* uoo_1, c
   const size_t IE = h->IE, JE = h->JE, KE = h->KE;
   const size_t u3 = (IE - h->i_start + 1) * JE * KE, v3 = IE * (JE - h->j_start + 1) * KE, w3 = IE * JE * (KE + 1);
   hipStream_t st = h->stream;
-  hipError_t e = hipMemcpyAsync(h->d_uoo, uoo, u3 * 8, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(h->d_uoo_1, uoo_1, u3 * 8, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(h->d_voe, voe, v3 * 8, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(h->d_voe_1, voe_1, v3 * 8, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(h->d_wno, wno, w3 * 8, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(h->d_wno_1, wno_1, w3 * 8, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(h->d_zo, zo, IE * JE * 8, hipMemcpyHostToDevice, st);
+  const XferPiece in[] = {xfer_flat(h->d_uoo, uoo, u3 * 8), xfer_flat(h->d_uoo_1, uoo_1, u3 * 8),
+                          xfer_flat(h->d_voe, voe, v3 * 8), xfer_flat(h->d_voe_1, voe_1, v3 * 8),
+                          xfer_flat(h->d_wno, wno, w3 * 8), xfer_flat(h->d_wno_1, wno_1, w3 * 8),
+                          xfer_flat(h->d_zo, zo, IE * JE * 8)};
+  hipError_t e = xfer_to_device(h->opts.device, st, in, 7);
   // DIVG into the Fortran staging array; with the bottom solve, PNH_bot and the corrections of DIVG
   // (ComputeRHS with CG2D4NONHY); then b = DIVG*WETO exactly as orctm_nh_set_rhs forms it
   if (e == hipSuccess) e = launch_divergence(st, h->ocv, h->d_fort);
@@ -1761,10 +1759,8 @@ int orctm_nh_divergence(orctm_nh_t* h, const double* uoo, const double* uoo_1, c
     e = launch_rhs(st, h->ctx.d_sys, h->ctx.d_tiles, h->ctx.ntiles, 1, h->d_fort, h->IE, h->JE);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (e == hipSuccess && divg) {
-    for (size_t k = 0; k < KE && e == hipSuccess; ++k) {
-      const size_t off = 1 + IE * (1 + JE * k);
-      e = hipMemcpy2D(divg + off, IE * 8, h->d_fort + off, IE * 8, (IE - 2) * 8, JE - 2, hipMemcpyDeviceToHost);
-    }
+    const XferPiece out = xfer_interior(h->d_fort + 1 + IE, divg, h->IE, h->JE, h->KE, IE, IE * JE);
+    e = xfer_to_host(h->opts.device, st, &out, 1);
   }
   return e == hipSuccess ? bot_status : map_err(e);
 }
@@ -1811,16 +1807,14 @@ int orctm_nh_project(orctm_nh_t* h, double* pnh, double* uoo, double* voe, doubl
   const size_t p3 = IE * JE * KE, u3 = (IE - h->i_start + 1) * JE * KE, v3 = IE * (JE - h->j_start + 1) * KE,
                w3 = IE * JE * (KE + 1);
   hipStream_t st = h->stream;
-  hipError_t e = hipMemcpyAsync(h->d_fort, pnh, p3 * 8, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(h->d_uoo, uoo, u3 * 8, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(h->d_voe, voe, v3 * 8, hipMemcpyHostToDevice, st);
+  const XferPiece in[] = {xfer_flat(h->d_fort, pnh, p3 * 8), xfer_flat(h->d_uoo, uoo, u3 * 8),
+                          xfer_flat(h->d_voe, voe, v3 * 8)};
+  hipError_t e = xfer_to_device(h->opts.device, st, in, 3);
   if (e == hipSuccess)
     e = launch_project(st, h->ocv, h->sys.p64, h->pitch, h->plane, h->d_fort, h->d_uoo, h->d_voe, h->d_wno);
-  if (e == hipSuccess) e = hipMemcpyAsync(pnh, h->d_fort, p3 * 8, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(uoo, h->d_uoo, u3 * 8, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(voe, h->d_voe, v3 * 8, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(wno, h->d_wno, w3 * 8, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  const XferPiece out[] = {xfer_flat(h->d_fort, pnh, p3 * 8), xfer_flat(h->d_uoo, uoo, u3 * 8),
+                           xfer_flat(h->d_voe, voe, v3 * 8), xfer_flat(h->d_wno, wno, w3 * 8)};
+  if (e == hipSuccess) e = xfer_to_host(h->opts.device, st, out, 4);
   return map_err(e);
 }
 

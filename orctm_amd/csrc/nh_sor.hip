@@ -23,6 +23,7 @@
 #include "nh_lock.h"
 #include "nh_ocv.h"
 #include "nh_sor_tb.h"
+#include "nh_xfer.h"
 
 namespace onh {
 namespace {
@@ -190,6 +191,7 @@ void sor_free(orctm_nh_sor_t* s) {
   if (s->stream) hipStreamDestroy(s->stream);
   for (void* p : s->allocs) hipFree(p);
   s->allocs.clear();
+  xfer_release();
 }
 
 int sor_map(hipError_t e) {
@@ -314,6 +316,7 @@ int orctm_nh_sor_create(const orctm_nh_sor_grid_t* g, orctm_nh_sor_t** out) {
   if (hipSetDevice(g->device) != hipSuccess) return ORCTM_NH_ERR_NODEVICE;
   orctm_nh_sor_t* s = new (std::nothrow) orctm_nh_sor_t();
   if (!s) return ORCTM_NH_ERR_NOMEM;
+  xfer_retain();
   s->g = *g;
   SorDims& d = s->d;
   d.IE = g->ie;
@@ -397,11 +400,10 @@ int orctm_nh_troneu(orctm_nh_sor_t* s, const double* u1o, const double* uzo, con
   const SorDims& d = s->d;
   const size_t p2 = (size_t)d.IE * d.JE, u2 = (size_t)d.NU * d.JE, v2 = (size_t)d.IE * (d.JE - d.JS + 1);
   hipStream_t st = s->stream;
-  hipError_t e = hipMemcpyAsync(s->a.u1o, u1o, u2 * 8, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(s->a.uzo, uzo, u2 * 8, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(s->a.v1e, v1e, v2 * 8, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(s->a.vze, vze, v2 * 8, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(s->a.b1o, b1o, p2 * 8, hipMemcpyHostToDevice, st);
+  const XferPiece in[] = {xfer_flat(s->a.u1o, u1o, u2 * 8), xfer_flat(s->a.uzo, uzo, u2 * 8),
+                          xfer_flat(s->a.v1e, v1e, v2 * 8), xfer_flat(s->a.vze, vze, v2 * 8),
+                          xfer_flat(s->a.b1o, b1o, p2 * 8)};
+  hipError_t e = xfer_to_device(s->g.device, st, in, 5);
   if (e == hipSuccess) e = hipEventRecord(s->ev0, st);
   if (e == hipSuccess) {
     const long long nb = (long long)(d.IE - d.IS) * (d.JE - d.JS);
@@ -414,9 +416,8 @@ int orctm_nh_troneu(orctm_nh_sor_t* s, const double* u1o, const double* uzo, con
   }
   if (e == hipSuccess && s->graph) e = hipGraphLaunch(s->graph, st);
   if (e == hipSuccess) e = hipEventRecord(s->ev1, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(z1o, s->a.z1o, p2 * 8, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(b1o, s->a.b1o, p2 * 8, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  const XferPiece out[] = {xfer_flat(s->a.z1o, z1o, p2 * 8), xfer_flat(s->a.b1o, b1o, p2 * 8)};
+  if (e == hipSuccess) e = xfer_to_host(s->g.device, st, out, 2);
   if (e == hipSuccess && device_ms) {
     float ms = 0.f;
     e = hipEventElapsedTime(&ms, s->ev0, s->ev1);

@@ -1,0 +1,245 @@
+// nh_xfer.cpp -- bulk transfers through pinned chunks (nh_xfer.h).
+#include "nh_xfer.h"
+
+#include <string.h>
+
+#include <algorithm>
+#include <atomic>
+#include <mutex>
+#include <system_error>
+#include <thread>
+
+#include "nh_lock.h"
+
+namespace onh {
+namespace {
+
+struct Stage {
+  std::mutex mu;  // held for a transfer; taken after device_lock() where both are
+  int device = -1;
+  char* buf[kXferWorkers][2] = {};
+  hipEvent_t ev[kXferWorkers][2] = {};
+};
+
+constexpr int kStages = 16;  // device ordinals beyond share them
+Stage g_stage[kStages];
+std::mutex g_count_mu;
+int g_handles = 0;
+
+bool made(const Stage& s, int workers, int device) {
+  if (s.device != device) return false;
+  for (int w = 0; w < workers; ++w)
+    for (int q = 0; q < 2; ++q)
+      if (!s.buf[w][q] || !s.ev[w][q]) return false;
+  return true;
+}
+
+void drop(Stage& s) {
+  for (int w = 0; w < kXferWorkers; ++w)
+    for (int q = 0; q < 2; ++q) {
+      if (s.ev[w][q]) hipEventDestroy(s.ev[w][q]);
+      if (s.buf[w][q]) hipHostFree(s.buf[w][q]);
+      s.ev[w][q] = nullptr;
+      s.buf[w][q] = nullptr;
+    }
+  s.device = -1;
+}
+
+hipError_t make(Stage& s, int workers, int device) {
+  if (s.device != device) drop(s);
+  s.device = device;
+  for (int w = 0; w < workers; ++w)
+    for (int q = 0; q < 2; ++q) {
+      hipError_t e = hipSuccess;
+      if (!s.buf[w][q]) {
+        void* p = nullptr;
+        e = hipHostMalloc(&p, kXferChunk, hipHostMallocDefault);
+        s.buf[w][q] = static_cast<char*>(p);
+      }
+      if (e == hipSuccess && !s.ev[w][q]) e = hipEventCreateWithFlags(&s.ev[w][q], hipEventDisableTiming);
+      if (e != hipSuccess) return e;
+    }
+  return hipSuccess;
+}
+
+struct Chunk {
+  const XferPiece* p = nullptr;
+  size_t off = 0, len = 0;  // bytes of the piece
+};
+
+struct Plan {
+  const XferPiece* p;
+  int n;
+  size_t step;                    // bytes of a chunk, a multiple of a double
+  size_t first[kXferPieces + 1];  // chunk number at which a piece begins
+  Plan(const XferPiece* pieces, int count, size_t chunk) : p(pieces), n(count), step(chunk) {
+    first[0] = 0;
+    for (int q = 0; q < n; ++q) first[q + 1] = first[q] + (p[q].bytes() + step - 1) / step;
+  }
+  size_t chunks() const { return first[n]; }
+  Chunk chunk(size_t k) const {
+    int q = 0;
+    while (k >= first[q + 1]) ++q;
+    const size_t off = (k - first[q]) * step;
+    return Chunk{p + q, off, std::min(step, p[q].bytes() - off)};
+  }
+};
+
+// The host half of a chunk.
+void host_copy(const Chunk& c, char* buf, bool to_host) {
+  const XferPiece& p = *c.p;
+  for (size_t done = 0; done < c.len;) {
+    const size_t at = c.off + done, row = at / p.row_bytes, in = at % p.row_bytes;
+    const size_t m = std::min(p.row_bytes - in, c.len - done);
+    char* h = p.host + row / p.rows * p.plane_stride + row % p.rows * p.row_stride + in;
+    if (to_host) memcpy(h, buf + done, m);
+    else memcpy(buf + done, h, m);
+    done += m;
+  }
+}
+
+hipError_t device_half(const Chunk& c, char* buf, bool to_host, hipStream_t st) {
+  const XferPiece& p = *c.p;
+  if (!p.dev_pitch)
+    return to_host ? hipMemcpyAsync(buf, p.dev + c.off, c.len, hipMemcpyDeviceToHost, st)
+                   : hipMemcpyAsync(p.dev + c.off, buf, c.len, hipMemcpyHostToDevice, st);
+  const size_t w = sizeof(double);
+  return launch_pack(st, reinterpret_cast<const double*>(p.dev), p.dev_pitch, p.dev_plane, p.row_bytes / w, p.rows,
+                     c.off / w, c.len / w, reinterpret_cast<double*>(buf));
+}
+
+// One worker: chunks from the common counter through its two buffers. Every copy that it issued has
+// finished when it returns.
+hipError_t work(Stage& s, int w, const Plan& plan, std::atomic<size_t>& next, bool to_host, hipStream_t st) {
+  hipError_t err = hipSuccess;
+  Chunk held[2];
+  bool pending[2] = {false, false};
+  auto settle = [&](int q) {
+    if (!pending[q]) return;
+    pending[q] = false;
+    const hipError_t e = hipEventSynchronize(s.ev[w][q]);
+    if (err == hipSuccess) err = e;
+    if (to_host && e == hipSuccess) host_copy(held[q], s.buf[w][q], true);
+  };
+  const size_t n = plan.chunks();
+  int q = 0;
+  for (size_t k = next++; k < n && err == hipSuccess; k = next++) {
+    settle(q);
+    held[q] = plan.chunk(k);
+    if (!to_host) host_copy(held[q], s.buf[w][q], false);
+    hipError_t e = device_half(held[q], s.buf[w][q], to_host, st);
+    if (e == hipSuccess) e = hipEventRecord(s.ev[w][q], st);
+    if (e == hipSuccess) {
+      pending[q] = true;
+    } else {
+      hipStreamSynchronize(st);  // a copy without an event may still use the buffer
+      err = e;
+    }
+    q ^= 1;
+    if (to_host) settle(q);  // the chunk before, while this one is on its way
+  }
+  settle(q);
+  settle(q ^ 1);
+  return err;
+}
+
+hipError_t transfer(int device, hipStream_t st, const XferPiece* p, int n, bool to_host) {
+  if (n < 0 || n > kXferPieces) return hipErrorInvalidValue;
+  size_t bytes = 0;
+  bool flat = true;
+  for (int q = 0; q < n; ++q) {
+    bytes += p[q].bytes();
+    flat = flat && p[q].rows * p[q].planes == 1 && !p[q].dev_pitch;
+  }
+  if (flat && bytes < (to_host ? kXferDirectHost : kXferDirectDevice)) {
+    hipError_t e = hipSuccess;
+    for (int q = 0; q < n && e == hipSuccess; ++q)
+      e = to_host ? hipMemcpyAsync(p[q].host, p[q].dev, p[q].bytes(), hipMemcpyDeviceToHost, st)
+                  : hipMemcpyAsync(p[q].dev, p[q].host, p[q].bytes(), hipMemcpyHostToDevice, st);
+    const hipError_t es = hipStreamSynchronize(st);
+    return e != hipSuccess ? e : es;
+  }
+  const size_t part = (bytes / 12 + 7) / 8 * 8;
+  const Plan plan(p, n, to_host ? std::min(std::max(part, kXferChunk / 8), kXferChunk) : kXferChunk);
+  if (plan.chunks() == 0) return hipSuccess;
+  const int want = bytes >= kXferThreaded ? (int)std::min<size_t>(kXferWorkers, plan.chunks()) : 1;
+  Stage& s = g_stage[(unsigned)device % kStages];
+  std::unique_lock<std::mutex> lk(s.mu);
+  while (!made(s, want, device)) {  // allocates: not while another thread captures a graph
+    lk.unlock();
+    std::lock_guard<std::recursive_mutex> dev(device_lock());
+    lk.lock();
+    const hipError_t e = make(s, want, device);
+    if (e != hipSuccess) return e;
+  }
+  std::atomic<size_t> next{0};
+  hipError_t got[kXferWorkers] = {};
+  std::thread team[kXferWorkers];
+  for (int w = 1; w < want; ++w) {
+    try {
+      team[w] = std::thread([&, w] {
+        const hipError_t e = hipSetDevice(device);
+        got[w] = e == hipSuccess ? work(s, w, plan, next, to_host, st) : e;
+      });
+    } catch (const std::system_error&) {
+      break;  // no thread to be had: the others take its share
+    }
+  }
+  got[0] = work(s, 0, plan, next, to_host, st);
+  for (std::thread& t : team)
+    if (t.joinable()) t.join();
+  for (hipError_t e : got)
+    if (e != hipSuccess) return e;
+  return hipSuccess;
+}
+
+}  // namespace
+
+XferPiece xfer_flat(void* dev, const void* host, size_t bytes) {
+  XferPiece p;
+  p.dev = static_cast<char*>(dev);
+  p.host = static_cast<char*>(const_cast<void*>(host));
+  p.row_bytes = bytes;
+  return p;
+}
+
+XferPiece xfer_interior(void* dev, const void* host, int IE, int JE, int KE, size_t dev_pitch, size_t dev_plane) {
+  XferPiece p;
+  p.dev = static_cast<char*>(dev);
+  p.host = static_cast<char*>(const_cast<void*>(host)) + sizeof(double) * (1 + (size_t)IE);
+  p.row_bytes = sizeof(double) * (size_t)(IE - 2);
+  p.rows = (size_t)(JE - 2);
+  p.planes = (size_t)KE;
+  p.row_stride = sizeof(double) * (size_t)IE;
+  p.plane_stride = p.row_stride * (size_t)JE;
+  p.dev_pitch = dev_pitch;
+  p.dev_plane = dev_plane;
+  return p;
+}
+
+hipError_t xfer_to_device(int device, hipStream_t st, const XferPiece* p, int n) {
+  for (int q = 0; q < n; ++q)
+    if (p[q].dev_pitch) return hipErrorInvalidValue;
+  return transfer(device, st, p, n, false);
+}
+
+hipError_t xfer_to_host(int device, hipStream_t st, const XferPiece* p, int n) {
+  return transfer(device, st, p, n, true);
+}
+
+void xfer_retain() {
+  std::lock_guard<std::mutex> lk(g_count_mu);
+  ++g_handles;
+}
+
+void xfer_release() {
+  std::lock_guard<std::recursive_mutex> dev(device_lock());
+  std::lock_guard<std::mutex> lk(g_count_mu);
+  if (--g_handles > 0) return;
+  for (Stage& s : g_stage) {
+    std::lock_guard<std::mutex> ls(s.mu);
+    if (s.device >= 0) drop(s);
+  }
+}
+
+}  // namespace onh
