@@ -32,6 +32,7 @@
 #include "nh_ocv.h"
 #include "nh_internal.h"
 #include "nh_pool.h"
+#include "nh_small.h"
 #include "nh_xfer.h"
 
 using namespace onh;
@@ -74,6 +75,10 @@ struct Ctx {
   bool own_stream = true;          // false: the stream belongs to the handle the context solves
   bool use_graphs = true;          // false: chunks are launched directly (short-lived serving cohorts)
   std::vector<Group> groups;       // inner-iteration tilings, one per tile height in use
+  bool small = false;              // the iterations run on 64-column rows (nh_small.h), not on the groups
+  SmallLaunch rows;
+  Tile* d_rows = nullptr;
+  void* d_inner2 = nullptr;        // second copies of the inner states (nh_small.hip)
   std::vector<int> heights;        // tile height of each system
   std::vector<int> tab;            // per system: 1 = ZW/ZP read from the table and window
   bool buf = false;                // the matvec kernel addresses memory through buffer descriptors
@@ -224,6 +229,9 @@ int alloc_state(orctm_nh_t* h) {
   SALLOC(pb, NP * es, void*);
   SALLOC(q, NP * es, void*);
   SALLOC(partials, 2 * (size_t)s.nslots * sizeof(double), double*);
+  // sums of nh_small.hip: per 64-column row, or per column where a block may take fewer
+  const size_t rows64 = (size_t)s.tiles_x * s.ny;
+  SALLOC(rowsum, 4 * rows64 * (rows64 * 64 <= (size_t)kSmallColumns ? 64 : 1) * es, void*);
   SALLOC(nbp, sizeof(double), double*);
 #undef SALLOC
   h->d_nb = s.nbp;
@@ -304,8 +312,10 @@ void ctx_destroy(Ctx& c) {
     pool_free(c.device, g.d_tiles);
     pool_free(c.device, g.d_pairs);
   }
+  pool_free(c.device, c.d_rows);
   pool_free(c.device, c.d_outer);
   pool_free(c.device, c.d_inner);
+  pool_free(c.device, c.d_inner2);
   pool_free_host(c.h_outer);
   pool_free_host(c.h_inner);
   pool_free(c.device, c.d_seeds);
@@ -339,6 +349,36 @@ hipError_t iter_fwd(Ctx& c, bool init, hipEvent_t e0 = nullptr, hipEvent_t e1 = 
   if (e1) HIPCHK(hipEventRecord(e1, c.stream));
   return launch_inner_reduce(c.stream, c.fp32, init ? PH_INIT : PH_FWD, c.d_sys, c.nsys);
 }
+
+// The first column update of an inner solve, and n iterations.
+hipError_t inner_start(Ctx& c) { return c.small ? small_begin(c.stream, c.rows) : iter_fwd(c, true); }
+
+hipError_t inner_run(Ctx& c, int n) {
+  if (c.small) return small_iterations(c.stream, c.rows, n);
+  for (int it = 0; it < n; ++it) {
+    HIPCHK(iter_bwd(c, 0));
+    HIPCHK(iter_fwd(c, false));
+  }
+  return hipSuccess;
+}
+
+// One iteration with events around the matvec and the column update.
+hipError_t inner_timed(Ctx& c, const hipEvent_t* ev) {
+  if (!c.small) {
+    HIPCHK(iter_bwd(c, 0, ev[0], ev[1]));
+    return iter_fwd(c, false, ev[2], ev[3]);
+  }
+  HIPCHK(hipEventRecord(ev[0], c.stream));
+  HIPCHK(small_matvec(c.stream, c.rows));
+  HIPCHK(hipEventRecord(ev[1], c.stream));
+  HIPCHK(hipEventRecord(ev[2], c.stream));
+  HIPCHK(small_update(c.stream, c.rows));
+  HIPCHK(hipEventRecord(ev[3], c.stream));
+  return small_finish(c.stream, c.rows);
+}
+
+// The first matvec of an inner solve (verification: q = C z, p = z).
+hipError_t inner_matvec(Ctx& c, int raw) { return c.small ? small_matvec(c.stream, c.rows) : iter_bwd(c, raw); }
 
 // ---- tile-height tuning --------------------------------------------------------------------------
 // The inner kernels run on 64 x h tiles, h in {4, 8, 12}. Small h gives more blocks (small systems
@@ -672,6 +712,55 @@ hipError_t ctx_heights(Ctx& c, const std::vector<Sys>& dev, const std::vector<in
 // 12% and lowers that of a 512x4x100 transect by 14%, whose launches fill a few dozen CUs.
 constexpr long long kTabMinCells = 1LL << 20;
 
+// How many 64-column rows a context may have for its iterations to run on blocks of columns (nh_small.h):
+// there they are bound by latency, and the blocks' own (one of 12 wavefronts a CU) is the shorter. Measured in us
+// per iteration, tiled against blocks, mixed / FP64: 512x4x100 (32 rows) 75 / 124 against 20 / 26; 128x128x30 (256)
+// 38 / 53 against 19 / 24; 192x160x35 (480) 49 / 70 against 32 / 56; 192x192x45 (576) 57 / 84 against 45 / 82;
+// 256x192x40 (768) 54 / 80 against 45 / 83.
+constexpr long long kSmallRows[2] = {512, 768};  // FP64, mixed
+// A single system of at most 64 rows takes blocks of 16 columns (up to 256 of them; 512x4x100 in blocks of 64:
+// 25 / 42 us); FP64 one of at most 128 rows and more than 56 levels blocks of 32 (1024x8x100: 43 against 61 us,
+// which has too many levels for the LDS of 64; 64x100x50: 32 against 31).
+constexpr long long kRows16 = 64, kRows32 = 128;
+constexpr int kLevels32 = 57;
+static_assert(kRows32 * 64 <= kSmallColumns, "the columns' sums are kept");
+
+// Whether the context's iterations run on rows of columns, and how. A forced tile height asks for the tiled
+// kernels.
+hipError_t ctx_rows(Ctx& c, const std::vector<Sys>& dev, const std::vector<int>& forced) {
+  long long rows = 0;
+  SmallLaunch& l = c.rows;
+  l.nz = 0;
+  for (int q = 0; q < c.nsys; ++q) {
+    if (forced[q] > 0) return hipSuccess;
+    rows += (long long)dev[q].tiles_x * dev[q].ny;
+    l.nz = std::max(l.nz, dev[q].nz);
+  }
+  if (rows > kSmallRows[c.fp32 ? 1 : 0]) return hipSuccess;
+  l.fp32 = c.fp32;
+  l.nsys = c.nsys;
+  l.one = c.nsys == 1;
+  l.sys = dev[0];
+  l.d_sys = c.d_sys;
+  l.wc = !l.one || rows > kRows32 ? 64 : rows <= kRows16 ? 16 : !c.fp32 && l.nz >= kLevels32 ? 32 : 64;
+  if (!small_fits(l.nz, c.fp32, l.wc)) return hipSuccess;
+  l.nblocks = (int)rows * (64 / l.wc);
+  if (!l.one) {
+    std::vector<Tile> nat;
+    for (int q = 0; q < c.nsys; ++q) order_into(nat, dev[q], q, 1);
+    const std::vector<Tile> ord = xcd_order(nat);
+    void* p = nullptr;
+    HIPCHK(pool_alloc(c.device, sizeof(Tile) * ord.size(), &p));
+    c.d_rows = static_cast<Tile*>(p);
+    HIPCHK(put_async(c.d_rows, ord.data(), sizeof(Tile) * ord.size(), c.stream));
+    HIPCHK(hipStreamSynchronize(c.stream));
+    l.d_rows = c.d_rows;
+  }
+  HIPCHK(small_setup(l));
+  c.small = true;
+  return hipSuccess;
+}
+
 // stream: the owning handle's stream for a single-system context, or nullptr for a context of its own
 // (a batch), which then creates one. Everything the build does is ordered on that stream.
 hipError_t ctx_build(Ctx& c, const std::vector<Sys>& systems, const std::vector<int>& forced,
@@ -713,6 +802,8 @@ hipError_t ctx_build(Ctx& c, const std::vector<Sys>& systems, const std::vector<
   HIPCHK(hipMemsetAsync(c.d_outer, 0, sizeof(Outer) * c.nsys, c.stream));
   HIPCHK(pool_alloc(device, inner_size(fp32) * c.nsys, &c.d_inner));
   HIPCHK(hipMemsetAsync(c.d_inner, 0, inner_size(fp32) * c.nsys, c.stream));
+  HIPCHK(pool_alloc(device, inner_size(fp32) * c.nsys, &c.d_inner2));
+  HIPCHK(hipMemsetAsync(c.d_inner2, 0, inner_size(fp32) * c.nsys, c.stream));
   HIPCHK(pool_alloc_host(sizeof(Outer) * c.nsys, &p));
   c.h_outer = static_cast<Outer*>(p);
   HIPCHK(pool_alloc_host(inner_size(fp32) * c.nsys, &c.h_inner));
@@ -725,6 +816,7 @@ hipError_t ctx_build(Ctx& c, const std::vector<Sys>& systems, const std::vector<
   for (int q = 0; q < c.nsys; ++q) {
     dev[q].outer = c.d_outer + q;
     dev[q].inner = static_cast<char*>(c.d_inner) + inner_size(fp32) * q;
+    dev[q].inner2 = static_cast<char*>(c.d_inner2) + inner_size(fp32) * q;
     const int mode = zw_table[q];
     dev[q].tab = dev[q].tab && (mode == 1 || (mode == 0 && c.cells >= kTabMinCells)) ? 1 : 0;
     c.tab[q] = dev[q].tab;
@@ -739,7 +831,8 @@ hipError_t ctx_build(Ctx& c, const std::vector<Sys>& systems, const std::vector<
   c.d_otiles = static_cast<Tile*>(p);
   if (c.n_otiles) HIPCHK(put_async(c.d_otiles, oord.data(), sizeof(Tile) * c.n_otiles, c.stream));
   HIPCHK(hipStreamSynchronize(c.stream));
-  return ctx_heights(c, dev, forced);
+  HIPCHK(ctx_heights(c, dev, forced));
+  return ctx_rows(c, dev, forced);
 }
 
 // n inner iterations (matvec + column update each). Runs of a power-of-two length are captured
@@ -747,19 +840,10 @@ hipError_t ctx_build(Ctx& c, const std::vector<Sys>& systems, const std::vector<
 // With kernel timing on, the same launches are issued directly with HIP events around each phase.
 hipError_t ctx_chunk(Ctx& c, int n) {
   if (c.prof) {
-    for (int it = 0; it < n; ++it) {
-      HIPCHK(iter_bwd(c, 0, c.kev[4 * it], c.kev[4 * it + 1]));
-      HIPCHK(iter_fwd(c, false, c.kev[4 * it + 2], c.kev[4 * it + 3]));
-    }
+    for (int it = 0; it < n; ++it) HIPCHK(inner_timed(c, &c.kev[4 * it]));
     return hipSuccess;
   }
-  if (!c.use_graphs) {
-    for (int it = 0; it < n; ++it) {
-      HIPCHK(iter_bwd(c, 0));
-      HIPCHK(iter_fwd(c, false));
-    }
-    return hipSuccess;
-  }
+  if (!c.use_graphs) return inner_run(c, n);
   for (int len = 1 << 30; len > 0; len >>= 1) {
     if (!(n & len)) continue;
     hipGraphExec_t& ge = c.graphs[len];
@@ -767,11 +851,7 @@ hipError_t ctx_chunk(Ctx& c, int n) {
       DEVLOCK;
       hipGraph_t g = nullptr;
       HIPCHK(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
-      hipError_t e = hipSuccess;
-      for (int it = 0; it < len && e == hipSuccess; ++it) {
-        e = iter_bwd(c, 0);
-        if (e == hipSuccess) e = iter_fwd(c, false);
-      }
+      hipError_t e = inner_run(c, len);
       hipError_t e2 = hipStreamEndCapture(c.stream, &g);
       if (e != hipSuccess) {
         if (g) hipGraphDestroy(g);
@@ -842,7 +922,7 @@ hipError_t ctx_solve(Ctx& c, float* ms) {
     bool any = false;
     for (int q = 0; q < c.nsys; ++q) any |= (c.h_outer[q].odone == RUN);
     if (!any) break;
-    HIPCHK(iter_fwd(c, true));
+    HIPCHK(inner_start(c));
     std::fill(c.iter_seen.begin(), c.iter_seen.end(), 0);
     // every inner solve ends within maxit iterations (device-side NOTCONV); the host bound on the
     // iterations issued only guarantees termination of this loop whatever the device flags say
@@ -1514,7 +1594,7 @@ int orctm_nh_inner_apply(orctm_nh_t* h, const void* x, void* y) {
       e = hipMemcpy(c.d_inner, &in, sizeof(in), hipMemcpyHostToDevice);
     }
   }
-  if (e == hipSuccess) e = iter_bwd(c, 1);
+  if (e == hipSuccess) e = inner_matvec(c, 1);
   if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
   if (e == hipSuccess) e = to_host_vec(h, y, h->sys.q, es);
   return map_err(e);
@@ -1537,8 +1617,8 @@ int orctm_nh_inner_precond(orctm_nh_t* h, const void* r, void* z, double* rho) {
   o.odone = RUN;
   hipError_t e = hipMemcpy(c.d_outer, &o, sizeof(o), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = to_device_vec(h, h->sys.r, r, es);
-  if (e == hipSuccess) e = iter_fwd(c, true);
-  if (e == hipSuccess) e = iter_bwd(c, 0);
+  if (e == hipSuccess) e = inner_start(c);
+  if (e == hipSuccess) e = inner_matvec(c, 0);
   if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
   if (e == hipSuccess) e = to_host_vec(h, z, h->sys.pb, es);
   if (e == hipSuccess && rho) {

@@ -97,6 +97,8 @@ struct Sys {
   double* partials;     // 2*nslots partial sums (summed by the reduction kernel in slot order)
   Outer* outer;
   void* inner;          // Inner<T>*
+  void* inner2;         // second copy of the inner state (launches of few columns, nh_small.hip)
+  void* rowsum;         // 2 x 2 x tiles_x*ny sums over the 64-column rows (the same launches)
   double* nbp;          // ||b||_2 of the resident right-hand side (written by the rhs kernel)
   const double* smaxp;  // max S of the system (written by the assembly)
   double rtol, rtol_inner;

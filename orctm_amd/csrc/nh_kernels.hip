@@ -10,145 +10,10 @@
 // Floating-point steps that the CPU oracle restates bit for bit are written with explicit fma and
 // are compiled with -ffp-contract=off (no other contraction): the assembly of the reference
 // operator (mo_petsc.f90:543-782), the FP64 matvec, the inner matvec and the line preconditioner.
-#include <math.h>
-
-#include <type_traits>
-
-#include "nh_kernels.h"
-#include "nh_flags.h"
+#include "nh_dev.h"
 #include "nh_xfer.h"
 
 namespace onh {
-
-__device__ __forceinline__ double fmad(double a, double b, double c) { return fma(a, b, c); }
-__device__ __forceinline__ float fmad(float a, float b, float c) { return fmaf(a, b, c); }
-
-// Pointers read from a Sys in memory are generic; casting them to the global address space lets the
-// compiler use global_load/global_store and count only vector-memory operations in its waits.
-template <typename T>
-using gptr = __attribute__((address_space(1))) T*;
-template <typename T>
-__device__ __forceinline__ gptr<T> G(const void* p) {
-  return (gptr<T>)(const_cast<void*>(p));
-}
-
-template <typename T>
-__device__ __forceinline__ T wave_sum(T v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-
-// Storage of the FP32 line-preconditioner factors: IEEE fp16 bits, normal range only (the rules of
-// the oracle's factor_round32): l with |l| < 2^-14 is stored as 0; invD is scaled by a power of two
-// per column (largest scaled value in [2^14, 2^15)) with magnitudes raised to at least 2^-14. The
-// rounding is done with integer operations (ties to even) so that it is the oracle's to the bit;
-// decoding is the exact fp16 -> fp32 conversion.
-__device__ __forceinline__ uint16_t half_bits(float v) {
-  const uint32_t u0 = __float_as_uint(v);
-  const uint32_t sgn = (u0 >> 16) & 0x8000u;
-  const float a = fabsf(v);
-  if (!(a < 65520.0f)) return isnan(v) ? (uint16_t)0x7E00u : (uint16_t)(sgn | 0x7C00u);
-  if (a == 0.0f) return (uint16_t)sgn;
-  const uint32_t u = (u0 + 0xFFFu + ((u0 >> 13) & 1u)) & 0xFFFFE000u;
-  const uint32_t e = ((u >> 23) & 0xFFu) - 112u;  // fp32 exponent bias 127 -> fp16 bias 15
-  return (uint16_t)(sgn | (e << 10) | ((u >> 13) & 0x3FFu));
-}
-
-__device__ __forceinline__ float half_val(uint16_t b) { return (float)__builtin_bit_cast(_Float16, b); }
-
-constexpr float kHalfMin = 6.103515625e-05f;  // 2^-14
-
-// Streaming accesses of the inner kernels: every value is touched once per launch and re-read only
-// by the next launch, a gigabyte or more later, so they carry the non-temporal hint (no cache
-// residency is expected; the stores do not evict lines other blocks still read).
-template <typename T>
-__device__ __forceinline__ T ld_nt(gptr<const T> p, size_t i) {
-  return __builtin_nontemporal_load(p + i);
-}
-template <typename T>
-__device__ __forceinline__ void st_nt(gptr<T> p, size_t i, T v) {
-  __builtin_nontemporal_store(v, p + i);
-}
-
-// Buffer-descriptor access (the matvec kernel's column march). A descriptor covers one array; a lane
-// addresses it by a 32-bit byte offset (its column's offset plus the level's). A lane that must not
-// touch memory takes an offset at or past kOob, beyond every array of at most kBufMaxBytes: the
-// hardware's range check then returns 0 for its load and drops its store. A whole wavefront is masked
-// by a descriptor of size 0. So every wavefront issues the same memory instructions on every path, and
-// the compiler's wait counts keep the loads of the next level in flight instead of draining them where
-// branches around loads and stores join.
-constexpr uint32_t kOob = 0x80000000u;
-static_assert(kBufMaxBytes <= kOob, "offsets of valid lanes stay below kOob");
-constexpr int kBufWord3 = 0x00020000;  // gfx9 descriptor word 3: 32-bit data format, untyped access
-using Rsrc = __amdgpu_buffer_rsrc_t;
-enum : int { kAuxNone = 0, kAuxNt = 2 };  // cache policy bits: none, non-temporal
-
-__device__ __forceinline__ Rsrc buf_of(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, kBufWord3);
-}
-template <typename E, int AUX>
-__device__ __forceinline__ E bld(Rsrc r, uint32_t vo) {
-  if constexpr (sizeof(E) == 2) {
-    return __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b16(r, vo, 0, AUX));
-  } else if constexpr (sizeof(E) == 4) {
-    return __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b32(r, vo, 0, AUX));
-  } else {
-    static_assert(sizeof(E) == 8, "2-, 4- or 8-byte elements");
-    return __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b64(r, vo, 0, AUX));
-  }
-}
-template <typename E>
-__device__ __forceinline__ void bst_nt(Rsrc r, uint32_t vo, E v) {
-  if constexpr (sizeof(E) == 4) {
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, vo, 0, kAuxNt);
-  } else {
-    static_assert(sizeof(E) == 8, "4- or 8-byte elements");
-    typedef unsigned int U2 __attribute__((ext_vector_type(2)));
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v), r, vo, 0, kAuxNt);
-  }
-}
-
-// Factor storage per inner precision: fp16 bits for FP32, the value itself for FP64.
-template <typename T>
-struct Fac {
-  using S = T;
-  __device__ static T dec(T v) { return v; }
-  __device__ static T ld(gptr<const S> p, size_t i) { return p[i]; }
-  __device__ static T ld_nt(gptr<const S> p, size_t i) { return onh::ld_nt(p, i); }
-};
-template <>
-struct Fac<float> {
-  using S = uint16_t;
-  __device__ static float dec(uint16_t v) { return half_val(v); }
-  __device__ static float ld(gptr<const uint16_t> p, size_t i) { return half_val(p[i]); }
-  __device__ static float ld_nt(gptr<const uint16_t> p, size_t i) { return half_val(onh::ld_nt(p, i)); }
-};
-
-// Sum of a and b over a block of NW wavefronts; valid in thread 0.
-template <typename T, int NW = NT / 64>
-__device__ __forceinline__ void block_sum2(T& a, T& b) {
-  __shared__ T sh[2 * NW];
-  a = wave_sum(a);
-  b = wave_sum(b);
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  __syncthreads();
-  if (l == 0) {
-    sh[w] = a;
-    sh[NW + w] = b;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    T sa = sh[0], sb = sh[NW];
-#pragma unroll
-    for (int q = 1; q < NW; ++q) {
-      sa += sh[q];
-      sb += sh[NW + q];
-    }
-    a = sa;
-    b = sb;
-  }
-}
 
 // Publishes the per-row sums of (a, b) of a block whose wavefront w (w < H) holds row j0 + w of its
 // tile, as totals over fixed groups of RG = 4 consecutive rows: group g = j / 4 of x-tile bx goes to
@@ -183,23 +48,6 @@ __device__ __forceinline__ void publish_rows(const Sys& s, int bx, int by, T a, 
   }
 }
 
-// Neighbour map of the DMDA: periodic wrap where cyclic, else validity (outside reads +0).
-__device__ __forceinline__ bool map_ij(int& i, int& j, int nx, int ny, int cx, int cy) {
-  if (cx) {
-    if (i < 0)
-      i += nx;
-    else if (i >= nx)
-      i -= nx;
-  }
-  if (cy) {
-    if (j < 0)
-      j += ny;
-    else if (j >= ny)
-      j -= ny;
-  }
-  return i >= 0 && i < nx && j >= 0 && j < ny;
-}
-
 // ------------------------------------------------------------------------------------------------
 // Assembly: compute_matrix (mo_petsc.f90:543-782), one thread per interior column.
 
@@ -224,75 +72,6 @@ __device__ __forceinline__ double dddwo(const FortranIn& f, int I, int J, int K)
   if (d0 == 0.0) return dm;
   return (dm + d0) / 2.0;
 }
-
-// One row of compute_matrix rebuilt from the compact form, in T arithmetic (double: the operations
-// of the assembly, bit for bit; float: the inner operator). c7: centre, W, E, N, S, U, D.
-// flags: bit 0 wet; bits 1-6 coupling present W E N S U D; bits 7-8 X_C variant (full, XUe*XP,
-// XUw*XP, 0); bits 9-10 Y_C variant (full, YVs*YP, YVn*YP, 0); bit 11 Z_C variant (full, ZW*ZP).
-template <typename T>
-__device__ __forceinline__ void row_coef(const T* cc, T zwk, T zwk1, T zpk, unsigned f, T* c7) {
-  const T xw = cc[0], xe = cc[1], yn = cc[2], ys = cc[3];
-  const unsigned xc = (f >> 7) & 3u, yc = (f >> 9) & 3u;
-  const T X_C = xc == 0 ? cc[4] : xc == 1 ? xe : xc == 2 ? xw : T(0);
-  const T Y_C = yc == 0 ? cc[5] : yc == 1 ? ys : yc == 2 ? yn : T(0);
-  const T Z_C = ((f >> 11) & 1u) ? zwk * zpk : (zwk + zwk1) * zpk;
-  c7[0] = -(X_C + Y_C + Z_C);
-  c7[1] = (f & (1u << 1)) ? xw : T(0);
-  c7[2] = (f & (1u << 2)) ? xe : T(0);
-  c7[3] = (f & (1u << 3)) ? yn : T(0);
-  c7[4] = (f & (1u << 4)) ? ys : T(0);
-  c7[5] = (f & (1u << 5)) ? zwk * zpk : T(0);
-  c7[6] = (f & (1u << 6)) ? zwk1 * zpk : T(0);
-}
-
-// ZW/ZP of one column from the per-level table and the column's 3-level window, and the column's flag
-// bits from its wet depths (Sys::tab).
-template <typename T>
-struct ZCol {
-  gptr<const T> tw, tp;
-  int kx;
-  T w0, w1, w2, p0, p1, p2;
-  int kc, kw, ke, kn, ks;
-  unsigned edge;
-  __device__ void load(gptr<const T> tw_, gptr<const T> tp_, const int* xk, gptr<const T> xw, gptr<const T> xp,
-                       const uint32_t* xf, size_t P, size_t off) {
-    tw = tw_;
-    tp = tp_;
-    kx = xk[off];
-    w0 = xw[off];
-    w1 = xw[P + off];
-    w2 = xw[2 * P + off];
-    p0 = xp[off];
-    p1 = xp[P + off];
-    p2 = xp[2 * P + off];
-    const uint32_t a = xf[off], b = xf[P + off], c = xf[2 * P + off];
-    kc = (int)(a & 0xffffu);
-    kw = (int)(a >> 16);
-    ke = (int)(b & 0xffffu);
-    kn = (int)(b >> 16);
-    ks = (int)(c & 0xffffu);
-    edge = c >> 16;
-  }
-  // flag bits of level m (0-based) of a column of nz levels
-  __device__ unsigned flag(int m, int nz) const { return derive_flags(m + 1, nz, kc, kw, ke, kn, ks, edge); }
-  __device__ T zw(int m) const {
-    const int d = m - kx;
-    return d == 0 ? w0 : d == 1 ? w1 : d == 2 ? w2 : tw[m];
-  }
-  __device__ T zp(int m) const {
-    const int d = m - kx;
-    return d == 0 ? p0 : d == 1 ? p1 : d == 2 ? p2 : tp[m];
-  }
-  // the window's value at level m where the window covers m, else t (the table's entry)
-  __device__ T zw_or(int m, T t) const {
-    const int d = m - kx;
-    return d == 0 ? w0 : d == 1 ? w1 : d == 2 ? w2 : t;
-  }
-  __device__ T zp_or(int m, T t) const {
-    const int d = m - kx;
-    return d == 0 ? p0 : d == 1 ? p1 : d == 2 ? p2 : t;
-  }
-};
 
 // The wet column's ZW/ZP (mo_petsc.f90:557-590 with DDPO = DZW on every level), with the assembly's
 // expressions, so that full columns reproduce the assembled values bit for bit. One thread.
@@ -511,15 +290,6 @@ __global__ __launch_bounds__(NT) void k_assemble(const Sys* __restrict__ systems
     if (bflag) atomicOr(bad, 1);
     if (isfinite(m)) atomicMax(smax_bits, (unsigned long long)__double_as_longlong(m));
   }
-}
-
-// Inner operator row C = S * (-A), S = DLXP*DLYP/ZP, in T arithmetic from the T copies.
-template <typename T>
-__device__ __forceinline__ void inner_row(const T* cc, T zwk, T zwk1, T zpk, unsigned f, T* c7) {
-  row_coef<T>(cc, zwk, zwk1, zpk, f, c7);
-  const T S = cc[6] / zpk;
-#pragma unroll
-  for (int q = 0; q < 7; ++q) c7[q] = S * (-c7[q]);
 }
 
 // Line preconditioner factorisation (per column), restated by orc_line_factor*: the tridiagonal of
@@ -1003,12 +773,8 @@ struct Fac2<float> {
 // the row sums are the same bits in either layout.
 template <typename T>
 __device__ __forceinline__ T half_row_sum(T v0, T v1) {
-#pragma unroll
-  for (int off = 16; off > 0; off >>= 1) {
-    v0 += __shfl_xor(v0, off, 64);
-    v1 += __shfl_xor(v1, off, 64);
-  }
-  return v0 + v1;
+  auto half = [](T v) { return fold_add<1>(fold_add<2>(fold_add<4>(fold_add<8>(fold_add<16>(v))))); };
+  return half(v0) + half(v1);
 }
 
 // publish_rows for a block of two tiles whose wavefront w holds row w of both, the first tile in lanes
@@ -1625,9 +1391,9 @@ __global__ __launch_bounds__(NT) void k_reduce(const Sys* __restrict__ systems) 
   }
   block_sum2(a, b);
   if (threadIdx.x != 0) return;
-  if (MODE == RED_NB) {
+  if constexpr (MODE == RED_NB) {
     *s.nbp = sqrt((double)a);
-  } else if (MODE == RED_RES) {
+  } else if constexpr (MODE == RED_RES) {
     // FP64 residual norm: convergence test and set-up of the next inner solve
     const double nb = o->nb;
     const bool zero = (nb == 0.0);
@@ -1658,53 +1424,21 @@ __global__ __launch_bounds__(NT) void k_reduce(const Sys* __restrict__ systems) 
     }
     o->odone = od;
     if (od != RUN) in->done = SKIP;
-  } else if (MODE == RED_INIT) {
-    const T rho = a, rr = b;
-    in->rho = rho;
-    in->rr0 = rr;
-    in->rr = rr;
-    in->iter = 0;
-    in->first = 1;
-    in->pbuf = 0;
-    in->xpend = 0;
-    in->beta = T(0);
-    if (rr == T(0))
-      in->done = CONVERGED;
-    else if (!(rho > T(0)) || !isfinite((double)rho) || !isfinite((double)rr))
-      in->done = BREAKDOWN;
-    else
-      in->done = RUN;
-    if (in->done == BREAKDOWN) o->odone = BREAKDOWN;
-  } else if (MODE == RED_FWD) {
-    const T rho = a, rr = b;
-    in->iter += 1;
+  } else if constexpr (MODE == RED_INIT) {
+    Inner<T> v = *in;
+    inner_begin(v, a, b);
+    *in = v;
+    if (v.done == BREAKDOWN) o->odone = BREAKDOWN;
+  } else if constexpr (MODE == RED_FWD) {
+    Inner<T> v = *in;
+    inner_after_update(v, a, b);
+    *in = v;
     o->inner_total += 1;
-    in->rr = rr;
-    int d = RUN;
-    if (rr <= in->tol2 * in->rr0)
-      d = CONVERGED;
-    else if (!(rho > T(0)) || !isfinite((double)rho) || !isfinite((double)rr))
-      d = BREAKDOWN;
-    else if (in->iter >= in->maxit)
-      d = NOTCONV;
-    else {
-      in->beta = rho / in->rho;
-      in->rho = rho;
-    }
-    in->first = 0;
-    in->pbuf ^= 1;
-    in->xpend = 1;  // x += alpha p of this iteration: applied by the next matvec or by k_refine
-    in->done = d;
   } else {  // RED_BWD
-    const T pq = a;
-    const T alpha = in->rho / pq;
-    in->pq = pq;
-    in->alpha = alpha;
-    in->xpend = 0;  // the matvec just applied the previous iteration's update
-    if (!(pq > T(0)) || !isfinite((double)alpha)) {
-      in->done = BREAKDOWN;
-      if (in->iter == 0) o->odone = BREAKDOWN;
-    }
+    Inner<T> v = *in;
+    inner_after_matvec(v, a);
+    *in = v;
+    if (v.done == BREAKDOWN && v.iter == 0) o->odone = BREAKDOWN;
   }
 }
 
