@@ -17,6 +17,7 @@
 
 #include <mutex>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/orctm_nh.h"
@@ -137,10 +138,11 @@ __global__ __launch_bounds__(NT) void k_sor_tb(TbGeom g, const double* __restric
   const int tid = threadIdx.x;
   K::load(tid, vx0, vy0, g, zin, b1o, ff, uf, vf, sorpar, lz, r);
   __syncthreads();
+  // away from odd-period seams a half-sweep reads one colour plane and writes the other: no barrier between
 #define ONH_HALF(C)                                  \
   do {                                               \
     K::template compute<C>(tid, sorpai, lz, r);      \
-    __syncthreads();                                 \
+    if (SEAM) __syncthreads();                       \
     K::template write<C>(tid, lz, r);                \
     __syncthreads();                                 \
   } while (0)
@@ -156,6 +158,123 @@ __global__ __launch_bounds__(NT) void k_sor_tb(TbGeom g, const double* __restric
   if (h < nh) ONH_HALF(0);
 #undef ONH_HALF
   K::store(tid, vx0, vy0, g, lz, zout);
+}
+
+// All sweeps of a surface that one CU holds, in one launch of one block: Z1O in LDS, split by colour (a cell's
+// neighbours lie in the other plane, consecutive lanes read consecutive words), the coefficients of a thread's M
+// cells of each colour in registers. A half-sweep is a few LDS reads and a barrier, where a blocked launch
+// costs its launch, a round trip of loads and the redundant rings: 514 x 6 took 583 us in 43 launches.
+// Periodic sides: the source's exchange after every half-sweep copies cells 2 and E-1 to the halo; here the thread
+// that updates such a cell writes the copy too (one per direction: at least two interior cells each way), after
+// one whole exchange that replaces the halo's initial values. Reads during a half-sweep see a neighbour's
+// value from before it: an interior cell's neighbours have the other parity of i + j, and so have halo copies
+// unless a period is odd (SEAM), where the new values wait for a barrier before they are written.
+constexpr int ONE_NT = 1024;
+constexpr size_t kOneLds = 150 * 1024;
+
+__host__ __device__ inline int one_half(int IE) { return (IE + 3) / 2; }  // cells of a colour in a row, at most
+
+inline size_t one_lds(int IE, int JE) { return sizeof(double) * 2 * (size_t)JE * one_half(IE); }
+// Cells of a colour per thread that the surface takes (1 to 3), 0: it does not run in one block.
+inline int one_cells(int IE, int JE, int cyc_x, int cyc_y) {
+  if ((cyc_x && IE < 4) || (cyc_y && JE < 4) || (long long)JE * IE > 1 << 20 || one_lds(IE, JE) > kOneLds) return 0;
+  const int m = ((JE - 2) * ((IE - 1) / 2) + ONE_NT - 1) / ONE_NT;
+  return m <= 3 ? m : 0;
+}
+
+template <int M, bool SEAM>
+__global__ __launch_bounds__(ONE_NT) void k_sor_one(SorDims d, SorArrays a, int cyc_x, int cyc_y, int iterations,
+                                                    double sorpar, double sorpai) {
+  extern __shared__ double zs[];
+  const int IE = d.IE, JE = d.JE, H = one_half(IE), PL = JE * H;
+  auto at = [&](int i, int j) { return ((i + j) & 1) * PL + (j - 1) * H + (i >> 1); };
+  for (int n = threadIdx.x; n < IE * JE; n += ONE_NT) {  // troneu.f90:67-101
+    const int i = 1 + n % IE, j = 1 + n / IE;
+    const bool edge = i == 1 || i == IE || j == 1 || j == JE;
+    zs[at(i, j)] = edge ? a.b1o[d.p2(i, j)] / a.xx[d.p2(i, j)] : 0.0;
+  }
+  struct Cell {
+    double b, w, ue, uw, vn, vs;
+    int own, east;  // LDS places of the cell and of its eastern neighbour (the western one lies before that)
+    int dx, dy;     // places of the halo copies, -1: none
+  };
+  Cell c[2][M];
+  const int HR = (IE - 1) / 2;
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const int e = threadIdx.x + ONE_NT * m, j = 2 + e / HR, i = 2 + ((j + q) & 1) + 2 * (e % HR);
+      Cell& k = c[q][m];
+      k.own = -1;
+      if (j > JE - 1 || i > IE - 1) continue;
+      k.own = at(i, j);
+      k.east = at(i + 1, j);
+      k.b = a.b1o[d.p2(i, j)];
+      k.w = sorpar * a.ff[d.p2(i, j)];
+      k.ue = a.uf[d.u2(i, j)];
+      k.uw = a.uf[d.u2(i - 1, j)];
+      k.vn = a.vf[d.v2(i, j)];
+      k.vs = a.vf[d.v2(i, j - 1)];
+      k.dx = !cyc_x ? -1 : i == 2 ? at(IE, j) : i == IE - 1 ? at(1, j) : -1;
+      k.dy = !cyc_y ? -1 : j == 2 ? at(i, JE) : j == JE - 1 ? at(i, 1) : -1;
+    }
+  __syncthreads();
+  auto half = [&](const Cell* cs, bool copies) {
+    double z[M];
+    auto write = [&](int m) {
+      const Cell& k = cs[m];
+      zs[k.own] = z[m];
+      if (copies && k.dx >= 0) zs[k.dx] = z[m];
+      if (copies && k.dy >= 0) zs[k.dy] = z[m];
+    };
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const Cell& k = cs[m];
+      if (k.own < 0) continue;
+      const int e = k.east, o = k.own < PL ? k.own + PL : k.own - PL;  // own column in the other plane
+      const double s = k.b + k.ue * zs[e] + k.uw * zs[e - 1] + k.vn * zs[o + H] + k.vs * zs[o - H];
+      z[m] = k.w * s + sorpai * zs[k.own];
+      if (!SEAM) write(m);
+    }
+    __syncthreads();
+    if (SEAM) {
+#pragma unroll
+      for (int m = 0; m < M; ++m)
+        if (cs[m].own >= 0) write(m);
+      __syncthreads();
+    }
+  };
+  auto exchange = [&] {
+    if (cyc_x) {
+      for (int j = 1 + threadIdx.x; j <= JE; j += ONE_NT) {
+        const double lo = zs[at(2, j)], hi = zs[at(IE - 1, j)];
+        zs[at(1, j)] = hi;
+        zs[at(IE, j)] = lo;
+      }
+      __syncthreads();
+    }
+    if (cyc_y) {
+      for (int i = 1 + threadIdx.x; i <= IE; i += ONE_NT) {
+        const double lo = zs[at(i, 2)], hi = zs[at(i, JE - 1)];
+        zs[at(i, 1)] = hi;
+        zs[at(i, JE)] = lo;
+      }
+      __syncthreads();
+    }
+  };
+  half(c[0], false);
+  exchange();
+  half(c[1], true);
+  for (int it = 1; it < iterations; ++it) {
+    half(c[0], true);
+    half(c[1], true);
+  }
+  exchange();  // the corners
+  for (int n = threadIdx.x; n < IE * JE; n += ONE_NT) {
+    const int i = 1 + n % IE, j = 1 + n / IE;
+    a.z1o[d.p2(i, j)] = zs[at(i, j)];
+  }
 }
 
 constexpr int kTbDepths[] = {
@@ -177,6 +296,7 @@ struct orctm_nh_sor {
   hipStream_t stream = nullptr;
   hipGraphExec_t graph = nullptr;
   int depth = 0;     // half-sweeps per blocked launch
+  int one = 0;       // > 0: all sweeps in one launch, this many cells of a colour per thread (no graph)
   int launches = 0;  // kernel launches of the sweeps (the first half-sweep included)
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   std::mutex mu;
@@ -234,9 +354,35 @@ hipError_t sor_blocked(orctm_nh_sor_t* s, int& launches) {
   return e;
 }
 
+// An odd period in a cyclic direction puts cells of one colour side by side across the seam.
+bool has_seam(const orctm_nh_sor_t* s) {
+  return (s->g.cyclic_x && ((s->d.IE - 2) & 1)) || (s->g.cyclic_y && ((s->d.JE - 2) & 1));
+}
+
+// f(M, SEAM) for a surface that runs in one block.
+template <typename F>
+hipError_t by_one(const orctm_nh_sor_t* s, F&& f) {
+  using std::integral_constant;
+  const bool seam = has_seam(s);
+  switch (s->one) {
+    case 1: return seam ? f(integral_constant<int, 1>{}, std::true_type{}) : f(integral_constant<int, 1>{}, std::false_type{});
+    case 2: return seam ? f(integral_constant<int, 2>{}, std::true_type{}) : f(integral_constant<int, 2>{}, std::false_type{});
+    case 3: return seam ? f(integral_constant<int, 3>{}, std::true_type{}) : f(integral_constant<int, 3>{}, std::false_type{});
+  }
+  return hipErrorInvalidValue;
+}
+
+hipError_t sor_one(orctm_nh_sor_t* s) {
+  return by_one(s, [&](auto m, auto seam) {
+    hipLaunchKernelGGL((k_sor_one<decltype(m)::value, decltype(seam)::value>), dim3(1), dim3(ONE_NT),
+                       one_lds(s->d.IE, s->d.JE), s->stream, s->d, s->a, s->g.cyclic_x, s->g.cyclic_y, s->g.iterations,
+                       s->g.sorpar, 1. - s->g.sorpar);
+    return hipGetLastError();
+  });
+}
+
 hipError_t sor_sweeps(orctm_nh_sor_t* s, int T, int& launches) {
-  // an odd period in a cyclic direction puts cells of one colour side by side across the seam
-  const bool seam = (s->g.cyclic_x && ((s->d.IE - 2) & 1)) || (s->g.cyclic_y && ((s->d.JE - 2) & 1));
+  const bool seam = has_seam(s);
 #define X(TT, RX, RY, NT) \
   if (T == TT) return seam ? sor_blocked<TT, RX, RY, NT, true>(s, launches) : sor_blocked<TT, RX, RY, NT, false>(s, launches);
   ORCTM_SOR_TB_VARIANTS(X)
@@ -261,6 +407,15 @@ hipError_t sor_capture(orctm_nh_sor_t* s, int T, hipGraphExec_t* out, int& launc
 hipError_t sor_prepare(orctm_nh_sor_t* s, int want) {
   if (s->g.iterations < 1) return hipSuccess;
   hipError_t e = hipSuccess;
+  s->one = want ? 0 : one_cells(s->d.IE, s->d.JE, s->g.cyclic_x, s->g.cyclic_y);
+  if (s->one) {
+    s->depth = kTbDepths[sizeof(kTbDepths) / sizeof(kTbDepths[0]) - 1];
+    s->launches = 1;
+    return by_one(s, [&](auto m, auto seam) {
+      return hipFuncSetAttribute((const void*)&k_sor_one<decltype(m)::value, decltype(seam)::value>,
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)kOneLds);
+    });
+  }
   float best = 0.f;
   for (int T : kTbDepths) {
     if (want && T != want) continue;
@@ -403,14 +558,16 @@ int orctm_nh_troneu(orctm_nh_sor_t* s, const double* u1o, const double* uzo, con
   const XferPiece in[] = {xfer_flat(s->a.u1o, u1o, u2 * 8), xfer_flat(s->a.uzo, uzo, u2 * 8),
                           xfer_flat(s->a.v1e, v1e, v2 * 8), xfer_flat(s->a.vze, vze, v2 * 8),
                           xfer_flat(s->a.b1o, b1o, p2 * 8)};
-  hipError_t e = xfer_to_device(s->g.device, st, in, 5);
+  // the source recomputes B1O on J = J_start+1..JE, I = I_start+1..IE: all of it where both start at 0
+  hipError_t e = xfer_to_device(s->g.device, st, in, d.IS == 0 && d.JS == 0 ? 4 : 5);
   if (e == hipSuccess) e = hipEventRecord(s->ev0, st);
   if (e == hipSuccess) {
     const long long nb = (long long)(d.IE - d.IS) * (d.JE - d.JS);
     hipLaunchKernelGGL(k_b1o, dim3(nblk(nb)), dim3(SB), 0, st, d, s->a, s->g.cono, s->g.conn);
     e = hipGetLastError();
   }
-  if (e == hipSuccess) {
+  if (e == hipSuccess && s->one) e = sor_one(s);
+  if (e == hipSuccess && !s->one) {
     hipLaunchKernelGGL(k_z1o_init, dim3(nblk((long long)p2)), dim3(SB), 0, st, d, s->a);
     e = hipGetLastError();
   }

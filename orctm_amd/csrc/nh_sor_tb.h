@@ -17,9 +17,11 @@
 // result; across a cyclic seam with an odd period a neighbour can share the colour, and the source then
 // reads the halo copy, which also holds the value from before the half-sweep.
 //
-// Work split. A thread owns NP vertical pairs (x, 2p) and (x, 2p+1), one cell of each colour, so every
-// lane updates one cell per half-sweep; consecutive lanes own consecutive x, so the region loads and
-// the tile stores are contiguous rows. The LDS holds the region split by colour: plane (x + y) & 1,
+// Work split. A thread owns NP vertical pairs (x, 2p) and (x, 2p+1), one below the other, one cell of each
+// colour, so every lane updates one cell per half-sweep; consecutive lanes own consecutive x, so the region
+// loads and the tile stores are contiguous rows. VF(J-1) of a cell is VF(J) of the cell above it, which the
+// thread has loaded for all but its first pair, and UF(I-1) is UF(I) of the lane before (on the device, RX =
+// 64): 10.2 loads a pair instead of 14 (NP = 5), of the 72 MB that a launch over 1026 x 770 cells brought in. The LDS holds the region split by colour: plane (x + y) & 1,
 // row y >> 1, column x, padded by a row and a word on either side, so the four neighbours of a cell lie
 // in the other plane, consecutive lanes read consecutive words, and a lane's reads for all its pairs
 // are one base address plus constant offsets. B1O and SORPAR*FF of every cell sit beside them in LDS;
@@ -76,7 +78,7 @@ struct SorTb {
   static constexpr int PR = RY / 2;        // pair rows
   static constexpr int PL = RX * PR;       // cells per colour plane = pairs per region
   static constexpr int NP = PL / NT;       // pairs per thread
-  static constexpr int DP = NT / RX;       // pair rows between consecutive pairs of a thread
+  static constexpr int DP = 1;             // pair rows between consecutive pairs of a thread
   static constexpr int PAD = RX + 1;       // padding words before and after each plane
   static constexpr int PS = PL + 2 * PAD;  // plane stride
   static constexpr int BW = 2 * PS;        // start of the (B1O, SORPAR*FF) pairs, same plane order, no padding
@@ -111,6 +113,9 @@ struct SorTb {
     return (size_t)(i - 1) + (size_t)g.IE * (size_t)(j - g.JS);
   }
 
+  __host__ __device__ static int at_least_2(int v) { return v < 2 ? 2 : v; }
+  __host__ __device__ static int pair_row(int tid, int k) { return tid / RX * NP + k; }
+
   // Region origin (virtual coordinates of region cell (0, 0)) of tile t.
   __host__ __device__ static void origin(const TbGeom& g, int t, int& vx0, int& vy0) {
     vx0 = 2 + (t % g.tiles_x) * TXo - T;
@@ -126,10 +131,11 @@ struct SorTb {
     r.m0 = 0u;
     r.m1 = 0u;
     r.s0 = (vx0 + x + vy0) & 1;
+    TbCo co[NP][2];
+    double above = vf[v2(g, mi ? mi : 2, at_least_2(tb_map(vy0 + 2 * pair_row(tid, 0), g.JE, g.cyc_y)) - 1)];
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-      const int p = tid / RX + DP * k;
-      TbCo co[2];
+      const int p = pair_row(tid, k);
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         const int y = 2 * p + s;
@@ -142,20 +148,40 @@ struct SorTb {
         const int zi = in ? mi : 2, zj = in ? mj : 2, ci = upd ? mi : 2, cj = upd ? mj : 2;
         const double zv = zin[p2(g, zi, zj)];
         const double b = b1o[p2(g, ci, cj)], f = ff[p2(g, ci, cj)];
-        const double ue = uf[u2(g, ci, cj)], uw = uf[u2(g, ci - 1, cj)];
-        const double vn = vf[v2(g, ci, cj)], vs = vf[v2(g, ci, cj - 1)];
+        const double ue = uf[u2(g, zi, zj)], vn = vf[v2(g, zi, zj)];
+#if defined(__HIP_DEVICE_COMPILE__)
+        // lane 0 holds the region's first column, which is not updated
+        const double uw = RX == 64 ? __shfl_up(ue, 1, 64) : uf[u2(g, ci - 1, cj)];
+#else
+        const double uw = uf[u2(g, ci - 1, cj)];
+#endif
         r.z[k][s] = in ? zv : 0.0;
         lz[at(x, y)] = r.z[k][s];
         // SORPAR*FF(I,J) is the first product of the source's expression
         lz[bw(x, y)] = upd ? b : 0.0;
         lz[bw(x, y) + 1] = upd ? sorpar * f : 0.0;
-        co[s] = upd ? TbCo{ue, uw, vn, vs} : TbCo{0.0, 0.0, 0.0, 0.0};
+        co[k][s] = upd ? TbCo{ue, uw, vn, above} : TbCo{0.0, 0.0, 0.0, 0.0};
+        above = vn;
         const uint32_t bit = upd ? 1u << (2 * k + s) : 0u;
         if (((mi + mj) & 1) == 0) r.m0 |= bit;
         else r.m1 |= bit;
       }
-      r.c[0][k] = r.s0 ? co[1] : co[0];
-      r.c[1][k] = r.s0 ? co[0] : co[1];
+    }
+    if (g.cyc_x || g.cyc_y) {  // across a seam the lane before and the row above are columns IE-1, JE-1, not 1
+#pragma unroll
+      for (int k = 0; k < NP; ++k)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const int mj = tb_map(vy0 + 2 * pair_row(tid, k) + s, g.JE, g.cyc_y);
+          if (!(((r.m0 | r.m1) >> (2 * k + s)) & 1u)) continue;
+          if (mi == 2) co[k][s].uw = uf[u2(g, 1, mj)];
+          if (mj == 2) co[k][s].vs = vf[v2(g, mi, 1)];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      r.c[0][k] = r.s0 ? co[k][1] : co[k][0];
+      r.c[1][k] = r.s0 ? co[k][0] : co[k][1];
     }
     // the padding, read by the region's edge cells on the regular path (their results are discarded)
     for (int i = tid; i < 2 * PAD; i += NT) {
@@ -174,7 +200,7 @@ struct SorTb {
   // New values of this thread's cells of colour C, from the region as it stands (before the writes).
   template <int C>
   __host__ __device__ static void compute(int tid, double sorpai, const double* lz, Regs& r) {
-    const int x = tid % RX, p0 = tid / RX;
+    const int x = tid % RX, p0 = pair_row(tid, 0);
     if (!SEAM) {
       // The active cell of every pair is cell s; its pair partner (cell 1-s, the neighbour above for
       // s = 0 and below for s = 1) and its own value are in registers, the other vertical neighbour
@@ -221,7 +247,7 @@ struct SorTb {
 
   template <int C>
   __host__ __device__ static void write(int tid, double* lz, const Regs& r) {
-    const int x = tid % RX, p0 = tid / RX;
+    const int x = tid % RX, p0 = pair_row(tid, 0);
     const uint32_t m = C ? r.m1 : r.m0;
     if (!SEAM) {
       const int s = r.s0 ^ C, own = (x + s) & 1;
@@ -247,7 +273,7 @@ struct SorTb {
     if (x < T || x >= T + TXo || vx > g.IE - 1) return;
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-      const int p = tid / RX + DP * k;
+      const int p = pair_row(tid, k);
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         const int y = 2 * p + s, vy = vy0 + y;
@@ -258,12 +284,16 @@ struct SorTb {
 };
 
 // The half-sweeps per launch that are compiled, with their regions: T, RX, RY, threads (pairs per
-// thread = RX*RY/2/threads).
+// thread = RX*RY/2/threads). Blocks of 1024 threads (16 wavefronts a CU instead of 8) hide more of a half-sweep's LDS
+// latency where the registers allow them, two pairs a thread: T = 12 on 514 x 445 cells 0.637 -> 0.535 ms a call,
+// T = 4 0.75. Three pairs (64 x 96) spill. 64 x 80 at 512 threads stays for T = 6, 7: its tiles cover 1026 x 770
+// cells in one round of the 256 CUs, and a launch's 15 us there are 6 us of loads (205 KB a CU at the Infinity
+// Cache's rate), 0.9 us a half-sweep and the launch itself.
 #define ORCTM_SOR_TB_VARIANTS(X) \
-  X(4, 64, 32, 256)              \
+  X(4, 64, 32, 512)              \
   X(6, 64, 80, 512)              \
   X(7, 64, 80, 512)              \
-  X(8, 64, 64, 512)              \
-  X(12, 64, 64, 512)
+  X(8, 64, 64, 1024)             \
+  X(12, 64, 64, 1024)
 
 }  // namespace onh
