@@ -33,6 +33,7 @@
 #include "nh_internal.h"
 #include "nh_pool.h"
 #include "nh_small.h"
+#include "nh_stream.h"
 #include "nh_xfer.h"
 
 using namespace onh;
@@ -75,6 +76,11 @@ struct Ctx {
   bool own_stream = true;          // false: the stream belongs to the handle the context solves
   bool use_graphs = true;          // false: chunks are launched directly (short-lived serving cohorts)
   std::vector<Group> groups;       // inner-iteration tilings, one per tile height in use
+  bool stream_form = false;        // the groups run the kernels of nh_stream.h
+  Tile* d_opairs = nullptr;        // pairs of the 64 x kOuterRows tiles
+  int n_opairs = 0;
+  bool all_tab = true, any_wrap = false;  // every system reads the ZW/ZP table; some system is periodic along x
+  int nz = 0;                      // most levels of a system
   bool small = false;              // the iterations run on 64-column rows (nh_small.h), not on the groups
   SmallLaunch rows;
   Tile* d_rows = nullptr;
@@ -313,6 +319,7 @@ void ctx_destroy(Ctx& c) {
     pool_free(c.device, g.d_pairs);
   }
   pool_free(c.device, c.d_rows);
+  pool_free(c.device, c.d_opairs);
   pool_free(c.device, c.d_outer);
   pool_free(c.device, c.d_inner);
   pool_free(c.device, c.d_inner2);
@@ -333,10 +340,24 @@ hipError_t put_async(void* dst, const void* src, size_t bytes, hipStream_t st) {
   return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st);
 }
 
+StreamLaunch stream_launch(const Ctx& c) {
+  StreamLaunch l;
+  l.fp32 = c.fp32;
+  l.tab = c.all_tab;
+  l.wrap = c.any_wrap;
+  l.d_sys = c.d_sys;
+  l.d_tiles = c.d_otiles;
+  l.ntiles = c.n_otiles;
+  l.d_pairs = c.d_opairs;
+  l.npairs = c.n_opairs;
+  return l;
+}
+
 // One inner-iteration phase over every tile group, then the phase's per-system reduction. With e0/e1
 // given, events bracket the phase's kernels (not the reduction) for kernel timing.
 hipError_t iter_bwd(Ctx& c, int raw, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
   if (e0) HIPCHK(hipEventRecord(e0, c.stream));
+  if (c.stream_form) HIPCHK(stream_matvec(c.stream, stream_launch(c)));
   for (const Group& g : c.groups) HIPCHK(launch_bwd(c.stream, c.fp32, c.buf, g.h, c.d_sys, g.d_tiles, g.ntiles, raw));
   if (e1) HIPCHK(hipEventRecord(e1, c.stream));
   return launch_inner_reduce(c.stream, c.fp32, PH_BWD, c.d_sys, c.nsys);
@@ -344,6 +365,7 @@ hipError_t iter_bwd(Ctx& c, int raw, hipEvent_t e0 = nullptr, hipEvent_t e1 = nu
 
 hipError_t iter_fwd(Ctx& c, bool init, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
   if (e0) HIPCHK(hipEventRecord(e0, c.stream));
+  if (c.stream_form) HIPCHK(stream_update(c.stream, stream_launch(c), init));
   for (const Group& g : c.groups)
     HIPCHK(launch_fwd(c.stream, c.fp32, init, g.h, c.d_sys, g.d_tiles, g.ntiles, g.d_pairs, g.npairs));
   if (e1) HIPCHK(hipEventRecord(e1, c.stream));
@@ -705,11 +727,11 @@ hipError_t ctx_heights(Ctx& c, const std::vector<Sys>& dev, const std::vector<in
   return hipSuccess;
 }
 
-// Builds a context over the given systems (host Sys copies; outer/inner pointers are replaced by
-// the context's own contiguous arrays). forced[q]: tile height of system q, 0 = tuned.
 // Solve contexts of at least this many cells read ZW/ZP from the table by default (options.zw_table 0).
 // Measured on gfx950 with the table forced on and off: it raises the rate of a 1024x768x60 system by
-// 12% and lowers that of a 512x4x100 transect by 14%, whose launches fill a few dozen CUs.
+// 12% and lowers that of a 512x4x100 transect by 14%, whose launches fill a few dozen CUs. The streaming kernels
+// always do: it also tells them the columns' depths (192x160x24, 0.7 M cells, us per iteration with planes and with
+// the table: 36 and 31, FP64 45 and 34; 1024x100x6: 31 and 29, 38 and 34).
 constexpr long long kTabMinCells = 1LL << 20;
 
 // How many 64-column rows a context may have for its iterations to run on blocks of columns (nh_small.h):
@@ -718,6 +740,11 @@ constexpr long long kTabMinCells = 1LL << 20;
 // 38 / 53 against 19 / 24; 192x160x35 (480) 49 / 70 against 32 / 56; 192x192x45 (576) 57 / 84 against 45 / 82;
 // 256x192x40 (768) 54 / 80 against 45 / 83.
 constexpr long long kSmallRows[2] = {512, 768};  // FP64, mixed
+// Where the launches of many columns would run the kernels of nh_stream.h, FP64 changes over at one block a CU (us per
+// iteration, blocks against those): 128x128x30 (256 rows) 24 against 36; 192x128x35 (384) 48 against 42;
+// 192x160x35 (480) 52 against 43. Mixed at the same line as above: 192x192x45 (576) 44 against 49; 256x192x40 (768)
+// 44 against 44.
+constexpr long long kSmallRowsStream[2] = {256, 768};
 // A single system of at most 64 rows takes blocks of 16 columns (up to 256 of them; 512x4x100 in blocks of 64:
 // 25 / 42 us); FP64 one of at most 128 rows and more than 56 levels blocks of 32 (1024x8x100: 43 against 61 us,
 // which has too many levels for the LDS of 64; 64x100x50: 32 against 31).
@@ -725,26 +752,35 @@ constexpr long long kRows16 = 64, kRows32 = 128;
 constexpr int kLevels32 = 57;
 static_assert(kRows32 * 64 <= kSmallColumns, "the columns' sums are kept");
 
-// Whether the context's iterations run on rows of columns, and how. A forced tile height asks for the tiled
-// kernels.
-hipError_t ctx_rows(Ctx& c, const std::vector<Sys>& dev, const std::vector<int>& forced) {
-  long long rows = 0;
+// The kernels that the context's iterations run: blocks of columns (nh_small.h), the streaming ones (nh_stream.h), or
+// the tiled ones, which a forced tile height asks for, and which take what the streaming ones do not hold (more than
+// kStreamLevels levels, arrays past the reach of buffer descriptors).
+void ctx_form(Ctx& c, const std::vector<Sys>& systems, const std::vector<int>& forced) {
   SmallLaunch& l = c.rows;
-  l.nz = 0;
-  for (int q = 0; q < c.nsys; ++q) {
-    if (forced[q] > 0) return hipSuccess;
-    rows += (long long)dev[q].tiles_x * dev[q].ny;
-    l.nz = std::max(l.nz, dev[q].nz);
+  long long rows = 0;
+  c.nz = 0;
+  for (const Sys& s : systems) {
+    rows += (long long)s.tiles_x * s.ny;
+    c.nz = std::max(c.nz, s.nz);
+    c.any_wrap = c.any_wrap || s.cyc_x;
   }
-  if (rows > kSmallRows[c.fp32 ? 1 : 0]) return hipSuccess;
+  for (int h : forced)
+    if (h > 0) return;
+  const bool stream = c.buf && c.nz <= kStreamLevels;
+  l.nz = c.nz;
   l.fp32 = c.fp32;
   l.nsys = c.nsys;
   l.one = c.nsys == 1;
+  l.wc = !l.one || rows > kRows32 ? 64 : rows <= kRows16 ? 16 : !c.fp32 && l.nz >= kLevels32 ? 32 : 64;
+  l.nblocks = (int)std::min(rows, kSmallRows[1]) * (64 / l.wc);
+  c.small = rows <= (stream ? kSmallRowsStream : kSmallRows)[c.fp32 ? 1 : 0] && small_fits(l.nz, c.fp32, l.wc);
+  c.stream_form = stream && !c.small;
+}
+
+hipError_t ctx_rows(Ctx& c, const std::vector<Sys>& dev) {
+  SmallLaunch& l = c.rows;
   l.sys = dev[0];
   l.d_sys = c.d_sys;
-  l.wc = !l.one || rows > kRows32 ? 64 : rows <= kRows16 ? 16 : !c.fp32 && l.nz >= kLevels32 ? 32 : 64;
-  if (!small_fits(l.nz, c.fp32, l.wc)) return hipSuccess;
-  l.nblocks = (int)rows * (64 / l.wc);
   if (!l.one) {
     std::vector<Tile> nat;
     for (int q = 0; q < c.nsys; ++q) order_into(nat, dev[q], q, 1);
@@ -756,11 +792,11 @@ hipError_t ctx_rows(Ctx& c, const std::vector<Sys>& dev, const std::vector<int>&
     HIPCHK(hipStreamSynchronize(c.stream));
     l.d_rows = c.d_rows;
   }
-  HIPCHK(small_setup(l));
-  c.small = true;
-  return hipSuccess;
+  return small_setup(l);
 }
 
+// Builds a context over the given systems (host Sys copies; outer/inner pointers are replaced by
+// the context's own contiguous arrays). forced[q]: tile height of system q, 0 = chosen here.
 // stream: the owning handle's stream for a single-system context, or nullptr for a context of its own
 // (a batch), which then creates one. Everything the build does is ordered on that stream.
 hipError_t ctx_build(Ctx& c, const std::vector<Sys>& systems, const std::vector<int>& forced,
@@ -775,13 +811,16 @@ hipError_t ctx_build(Ctx& c, const std::vector<Sys>& systems, const std::vector<
   for (const Sys& s : systems) c.cells += (long long)s.nx * s.ny * s.nz;
   c.fp32 = fp32;
   c.check_every = check_every > 0 ? check_every : 16;
+  ctx_form(c, systems, forced);
   c.max_outer = max_outer;
   c.device = device;
   for (const Sys& s : systems) c.maxit = std::max(c.maxit, s.maxit);
   std::vector<Tile> nat, onat;
   for (int q = 0; q < c.nsys; ++q) order_into(nat, systems[q], q, TY);
   for (int q = 0; q < c.nsys; ++q) order_into(onat, systems[q], q, kOuterRows);
-  std::vector<Tile> ord = xcd_order(nat), oord = balanced_order(onat, systems);
+  std::vector<Tile> ord = xcd_order(nat), oord = balanced_order(onat, systems),
+                    opairs = balanced_order(pair_tiles(onat), systems);
+  c.n_opairs = (int)opairs.size();
   c.ntiles = (int)ord.size();
   c.n_otiles = (int)oord.size();
   if (stream) {
@@ -818,8 +857,9 @@ hipError_t ctx_build(Ctx& c, const std::vector<Sys>& systems, const std::vector<
     dev[q].inner = static_cast<char*>(c.d_inner) + inner_size(fp32) * q;
     dev[q].inner2 = static_cast<char*>(c.d_inner2) + inner_size(fp32) * q;
     const int mode = zw_table[q];
-    dev[q].tab = dev[q].tab && (mode == 1 || (mode == 0 && c.cells >= kTabMinCells)) ? 1 : 0;
+    dev[q].tab = dev[q].tab && (mode == 1 || (mode == 0 && (c.stream_form || c.cells >= kTabMinCells))) ? 1 : 0;
     c.tab[q] = dev[q].tab;
+    c.all_tab = c.all_tab && dev[q].tab;
   }
   HIPCHK(pool_alloc(device, sizeof(Sys) * c.nsys, &p));
   c.d_sys = static_cast<Sys*>(p);
@@ -829,10 +869,15 @@ hipError_t ctx_build(Ctx& c, const std::vector<Sys>& systems, const std::vector<
   if (c.ntiles) HIPCHK(put_async(c.d_tiles, ord.data(), sizeof(Tile) * c.ntiles, c.stream));
   HIPCHK(pool_alloc(device, sizeof(Tile) * std::max(c.n_otiles, 1), &p));
   c.d_otiles = static_cast<Tile*>(p);
+  HIPCHK(pool_alloc(device, sizeof(Tile) * std::max(c.n_opairs, 1), &p));
+  c.d_opairs = static_cast<Tile*>(p);
+  if (c.n_opairs) HIPCHK(put_async(c.d_opairs, opairs.data(), sizeof(Tile) * c.n_opairs, c.stream));
   if (c.n_otiles) HIPCHK(put_async(c.d_otiles, oord.data(), sizeof(Tile) * c.n_otiles, c.stream));
   HIPCHK(hipStreamSynchronize(c.stream));
-  HIPCHK(ctx_heights(c, dev, forced));
-  return ctx_rows(c, dev, forced);
+  if (c.small) HIPCHK(ctx_rows(c, dev));
+  if (c.stream_form) c.heights.assign(c.nsys, kOuterRows);
+  else HIPCHK(ctx_heights(c, dev, forced));
+  return hipSuccess;
 }
 
 // n inner iterations (matvec + column update each). Runs of a power-of-two length are captured
@@ -1116,6 +1161,7 @@ int create_device(orctm_nh_t* h, const orctm_nh_grid_t* g) {
   ALLOC(tp, (size_t)h->nz * sizeof(double), const double*);
   ALLOC(xk, (size_t)h->plane * sizeof(int), const int*);
   ALLOC(xf, 3 * (size_t)h->plane * sizeof(uint32_t), const uint32_t*);
+  ALLOC(use, (size_t)h->plane * sizeof(int), int*);
   ALLOC(xw, 3 * (size_t)h->plane * sizeof(double), const double*);
   ALLOC(xp, 3 * (size_t)h->plane * sizeof(double), const double*);
   if (h->fp32) {
@@ -1594,6 +1640,7 @@ int orctm_nh_inner_apply(orctm_nh_t* h, const void* x, void* y) {
       e = hipMemcpy(c.d_inner, &in, sizeof(in), hipMemcpyHostToDevice);
     }
   }
+  if (e == hipSuccess) e = launch_use_all(c.stream, h->sys);
   if (e == hipSuccess) e = inner_matvec(c, 1);
   if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
   if (e == hipSuccess) e = to_host_vec(h, y, h->sys.q, es);
@@ -1617,6 +1664,7 @@ int orctm_nh_inner_precond(orctm_nh_t* h, const void* r, void* z, double* rho) {
   o.odone = RUN;
   hipError_t e = hipMemcpy(c.d_outer, &o, sizeof(o), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = to_device_vec(h, h->sys.r, r, es);
+  if (e == hipSuccess) e = launch_use_all(c.stream, h->sys);
   if (e == hipSuccess) e = inner_start(c);
   if (e == hipSuccess) e = inner_matvec(c, 0);
   if (e == hipSuccess) e = hipStreamSynchronize(c.stream);

@@ -207,8 +207,12 @@ template <typename T>
 __device__ __forceinline__ void row_coef(const T* cc, T zwk, T zwk1, T zpk, unsigned f, T* c7) {
   const T xw = cc[0], xe = cc[1], yn = cc[2], ys = cc[3];
   const unsigned xc = (f >> 7) & 3u, yc = (f >> 9) & 3u;
-  const T X_C = xc == 0 ? cc[4] : xc == 1 ? xe : xc == 2 ? xw : T(0);
-  const T Y_C = yc == 0 ? cc[5] : yc == 1 ? ys : yc == 2 ? yn : T(0);
+  // one select after the other: a chain of ?: becomes branches, which empty the load pipeline
+  T X_C = xc == 2 ? xw : T(0), Y_C = yc == 2 ? yn : T(0);
+  X_C = xc == 1 ? xe : X_C;
+  X_C = xc == 0 ? cc[4] : X_C;
+  Y_C = yc == 1 ? ys : Y_C;
+  Y_C = yc == 0 ? cc[5] : Y_C;
   const T Z_C = ((f >> 11) & 1u) ? zwk * zpk : (zwk + zwk1) * zpk;
   c7[0] = -(X_C + Y_C + Z_C);
   c7[1] = (f & (1u << 1)) ? xw : T(0);
@@ -249,6 +253,31 @@ struct ZCol {
   }
   // flag bits of level m (0-based) of a column of nz levels
   __device__ unsigned flag(int m, int nz) const { return derive_flags(m + 1, nz, kc, kw, ke, kn, ks, edge); }
+  // Prepared for coef(): beyond the column's own wet depth a neighbour's plays no part.
+  __device__ void clamp() {
+    kw = min(kw, kc);
+    ke = min(ke, kc);
+    kn = min(kn, kc);
+    ks = min(ks, kc);
+  }
+  // row_coef() of level m from the wet depths themselves, without the flag word: the same values.
+  __device__ void coef(int m, const T* cc, T zwk, T zwk1, T zpk, T* c7) const {
+    const bool wet = m < kc, w = m < kw, e = m < ke, n = m < kn, s = m < ks, below = m + 1 < kc;
+    T X_C = e ? cc[1] : T(0), Y_C = s ? cc[3] : T(0);
+    const T xw = e ? cc[4] : cc[0], yn = s ? cc[5] : cc[2];
+    X_C = w ? xw : X_C;
+    Y_C = n ? yn : Y_C;
+    X_C = wet ? X_C : cc[4];
+    Y_C = wet ? Y_C : cc[5];
+    const T zs = zwk + zwk1, Z_C = (m > 0 && wet && !below ? zwk : zs) * zpk;
+    c7[0] = -(X_C + Y_C + Z_C);
+    c7[1] = w && (edge & 1u) ? cc[0] : T(0);
+    c7[2] = e && (edge & 2u) ? cc[1] : T(0);
+    c7[3] = n && (edge & 4u) ? cc[2] : T(0);
+    c7[4] = s && (edge & 8u) ? cc[3] : T(0);
+    c7[5] = m > 0 && wet ? zwk * zpk : T(0);
+    c7[6] = below ? zwk1 * zpk : T(0);
+  }
   __device__ T zw(int m) const {
     const int d = m - kx;
     return d == 0 ? w0 : d == 1 ? w1 : d == 2 ? w2 : tw[m];
@@ -260,11 +289,15 @@ struct ZCol {
   // the window's value at level m where the window covers m, else t (the table's entry)
   __device__ T zw_or(int m, T t) const {
     const int d = m - kx;
-    return d == 0 ? w0 : d == 1 ? w1 : d == 2 ? w2 : t;
+    t = d == 2 ? w2 : t;
+    t = d == 1 ? w1 : t;
+    return d == 0 ? w0 : t;
   }
   __device__ T zp_or(int m, T t) const {
     const int d = m - kx;
-    return d == 0 ? p0 : d == 1 ? p1 : d == 2 ? p2 : t;
+    t = d == 2 ? p2 : t;
+    t = d == 1 ? p1 : t;
+    return d == 0 ? p0 : t;
   }
 };
 
@@ -272,6 +305,14 @@ struct ZCol {
 template <typename T>
 __device__ __forceinline__ void inner_row(const T* cc, T zwk, T zwk1, T zpk, unsigned f, T* c7) {
   row_coef<T>(cc, zwk, zwk1, zpk, f, c7);
+  const T S = cc[6] / zpk;
+#pragma unroll
+  for (int q = 0; q < 7; ++q) c7[q] = S * (-c7[q]);
+}
+// The same from the wet depths (ZCol::clamp() applied).
+template <typename T>
+__device__ __forceinline__ void inner_row(const T* cc, T zwk, T zwk1, T zpk, int m, const ZCol<T>& z, T* c7) {
+  z.coef(m, cc, zwk, zwk1, zpk, c7);
   const T S = cc[6] / zpk;
 #pragma unroll
   for (int q = 0; q < 7; ++q) c7[q] = S * (-c7[q]);

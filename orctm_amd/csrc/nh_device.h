@@ -83,6 +83,9 @@ struct Sys {
   // (periodic or not on the domain edge); with `tab` set the kernels derive each cell's flag bits from
   // them instead of reading the flag plane (checked bit for bit against it at create)
   const uint32_t* xf;
+  // with `tab`: per column, the levels that the inner solve at hand works on (k_residual): the most wet levels
+  // and the deepest nonzero of r of the 16 columns around it. The other levels of r, x, z, p and q are 0 or unused.
+  int* use;
   const void* invD;     // line preconditioner 1/D_k: FP64, or fp16 bits scaled by dscale (FP32)
   const void* L;        // line preconditioner l_k: FP64, or fp16 bits (FP32)
   const float* dscale;  // FP32 only: per-column power of two that multiplies the stored invD

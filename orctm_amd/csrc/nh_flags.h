@@ -20,7 +20,6 @@ namespace onh {
 // coupling can exist. Bit 0 wet; bits 1-6 couplings W, E, N, S, U, D; bits 7-8 / 9-10 the X_C / Y_C
 // variant (1: west / north land, 2: east / south land, 3: both); bit 11 the bottom Z_C.
 ONH_HD unsigned derive_flags(int K, int KE, int kc, int kw, int ke, int kn, int ks, unsigned edge) {
-  if (K > kc) return 0u;
   const bool ww = K <= kw, we = K <= ke, wn = K <= kn, ws = K <= ks, below = K < kc && K != KE;
   unsigned fl = 1u;
   if (ww && (edge & 1u)) fl |= 1u << 1;
@@ -32,7 +31,8 @@ ONH_HD unsigned derive_flags(int K, int KE, int kc, int kw, int ke, int kn, int 
   const unsigned xc = !ww ? (we ? 1u : 3u) : (we ? 0u : 2u);
   const unsigned yc = !wn ? (ws ? 1u : 3u) : (ws ? 0u : 2u);
   const unsigned zc = (K != 1 && !below) ? 1u : 0u;
-  return fl | xc << 7 | yc << 9 | zc << 11;
+  fl |= xc << 7 | yc << 9 | zc << 11;
+  return K > kc ? 0u : fl;
 }
 
 // The 3 words of interior column (I, J) (1-based, halo'd Fortran indices) from WETO(IE,JE,KE):

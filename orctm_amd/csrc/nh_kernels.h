@@ -40,6 +40,10 @@ hipError_t launch_begin(hipStream_t st, bool fp32, const Sys* d_sys, int nsys);
 // registers, 8 waves per SIMD) runs on the set-up tiling, where it is faster (194 against 203 us).
 // h = kOuterRows or TY (the set-up tiling).
 constexpr int kOuterRows = 4;
+// Bytes of a row, in the inner solve's precision, whose columns share their count of levels in use (Sys::use): masked
+// stores then fill whole 64-byte pieces. 1024x768x60, FP32, us of matvec / column update: 220 / 156; with 32 bytes
+// 232 / 164.
+constexpr int kUseBytes = 64;
 // Each phase launch below is followed by its one-block-per-system reduction (nsys blocks).
 hipError_t launch_residual(hipStream_t st, bool fp32, int h, const Sys* d_sys, const Tile* d_tiles, int ntiles,
                            int nsys);
@@ -68,6 +72,7 @@ inline bool bwd_buffers_fit(const Sys& s, bool fp32) {
   return (unsigned long long)s.plane * (unsigned long long)s.nz * (fp32 ? 4ull : 8ull) <= kBufMaxBytes;
 }
 hipError_t launch_inner_reduce(hipStream_t st, bool fp32, InnerPhase ph, const Sys* d_sys, int nsys);
+hipError_t launch_use_all(hipStream_t st, const Sys& s);
 hipError_t launch_refine(hipStream_t st, bool fp32, int h, const Sys* d_sys, const Tile* d_tiles, int ntiles);
 // The 7 planes of the reference operator rebuilt from the compact form (verification entry point).
 hipError_t launch_materialize(hipStream_t st, const Sys* d_sys, const Tile* d_tiles, int ntiles, double* A);

@@ -174,6 +174,7 @@ __global__ __launch_bounds__(NT) void k_zflags(const Sys* __restrict__ systems, 
   xf[col] = w[0];
   xf[P + col] = w[1];
   xf[2 * P + col] = w[2];
+  s.use[col] = (int)(w[0] & 0xffffu);  // for the timing of tile heights, before the first residual
   gptr<const uint16_t> flg = G<const uint16_t>(s.flg);
   bool diff = false;
   for (int K = 1; K <= f.KE; ++K) diff = diff || flg[(size_t)(K - 1) * P + col] != flags_from_words(K, f.KE, w);
@@ -532,6 +533,7 @@ __global__ __launch_bounds__(64 * H) void k_residual(const Sys* __restrict__ sys
   const double gamma = 1.0 / (o->smax * o->nr_prev);
   const int i = t.bx * TX + (threadIdx.x & (TX - 1)), j = t.by * H + (threadIdx.x >> 6);
   double acc = 0.0, dummy = 0.0;
+  int use = 0;
   if (i < s.nx && j < s.ny) {
     const int nx = s.nx, ny = s.ny, nz = s.nz;
     const size_t col = (size_t)j * s.pitch + i, P = s.plane, IP = s.pitch;
@@ -553,6 +555,7 @@ __global__ __launch_bounds__(64 * H) void k_residual(const Sys* __restrict__ sys
       if (tab)
         zc.load(G<const double>(s.tw), G<const double>(s.tp), s.xk, G<const double>(s.xw), G<const double>(s.xp), s.xf,
                 P, col);
+      use = tab ? zc.kc : nz;
       double cc[7];
       load_col(s, col, cc);
       // horizontal neighbour columns (periodic wrap where cyclic; absent ones read this column and
@@ -597,7 +600,9 @@ __global__ __launch_bounds__(64 * H) void k_residual(const Sys* __restrict__ sys
         const double r = v.b - a;
         acc = fma(r, r, acc);
         const double S = cc[6] / v.zp;
-        st_nt<T>(rin, col + (size_t)k * P, (T)((S * (-r)) * gamma));
+        const T ri = (T)((S * (-r)) * gamma);
+        st_nt<T>(rin, col + (size_t)k * P, ri);
+        if (ri != T(0)) use = max(use, k + 1);
         xu = x0;
         x0 = xd;
         zwk = v.zw1;
@@ -613,7 +618,18 @@ __global__ __launch_bounds__(64 * H) void k_residual(const Sys* __restrict__ sys
       }
     }
   }
+  if (s.tab) {
+#pragma unroll
+    for (int m = 1; m < kUseBytes / (int)sizeof(T); m *= 2) use = max(use, __shfl_xor(use, m));
+    if (i < s.nx && j < s.ny) s.use[(size_t)j * s.pitch + i] = use;
+  }
   publish_rows<double, H, H>(s, t.bx, t.by, acc, dummy);
+}
+
+// Every level of every column in use (vectors the caller gives for the operator or the preconditioner alone).
+__global__ __launch_bounds__(NT) void k_use_all(int* use, size_t n, int nz) {
+  const size_t k = (size_t)blockIdx.x * NT + threadIdx.x;
+  if (k < n) use[k] = nz;
 }
 
 template <typename T, int H>
@@ -635,8 +651,9 @@ __global__ __launch_bounds__(64 * H) void k_refine(const Sys* __restrict__ syste
   gptr<const T> pl = G<const T>(in->pbuf ? s.pb : s.pa);
   gptr<double> p64 = G<double>(s.p64);
   const size_t col = (size_t)j * s.pitch + i;
+  const int nz = s.tab ? min(s.use[col], s.nz) : s.nz;  // below, x is 0
 #pragma unroll 4
-  for (int k = 0; k < s.nz; ++k) {
+  for (int k = 0; k < nz; ++k) {
     const size_t idx = col + (size_t)k * s.plane;
     const T xv = ld_nt<T>(x, idx);
     const T xk = pend ? fmad(alpha, ld_nt<T>(pl, idx), xv) : xv;
@@ -1565,6 +1582,12 @@ hipError_t launch_residual(hipStream_t st, bool fp32, int h, const Sys* d_sys, c
     return fp32 ? residual_h<float, TY>(st, d_sys, d_tiles, ntiles, nsys)
                 : residual_h<double, TY>(st, d_sys, d_tiles, ntiles, nsys);
   return hipErrorInvalidValue;
+}
+
+hipError_t launch_use_all(hipStream_t st, const Sys& s) {
+  const size_t n = s.plane;
+  hipLaunchKernelGGL(k_use_all, dim3((unsigned)((n + NT - 1) / NT)), dim3(NT), 0, st, s.use, n, s.nz);
+  return hipGetLastError();
 }
 
 hipError_t launch_refine(hipStream_t st, bool fp32, int h, const Sys* d_sys, const Tile* d_tiles, int ntiles) {
