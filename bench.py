@@ -59,6 +59,28 @@ def fwd_bytes(cells, columns, W):
     return cells * (4 * W + 2 * F) + (columns * 4 if W == 4 else 0)
 
 
+# The streaming kernels, which run the launches of many columns unless a tile height is forced, work on the levels in
+# use: a column's wet depth, made equal over 64 bytes of a row. k_matvec reads z, p_old, x and writes p, q, x there;
+# per column the 7 products, the window, the wet depths and the levels in use. k_update reads r, q, l, invD and writes
+# r, z; per column the levels in use and, in FP32, the scale of invD.
+def cells_in_use(g, W):
+    depth = (np.asarray(g.weto)[1:-1, 1:-1, :] == 1.0).sum(axis=2)
+    nx, n = depth.shape[0], 64 // W
+    pad = np.zeros(((nx + n - 1) // n * n, depth.shape[1]), dtype=np.int64)
+    pad[:nx] = depth
+    deepest = np.repeat(pad.reshape(-1, n, pad.shape[1]).max(axis=1), n, axis=0)[:nx]
+    return int(deepest.sum())
+
+
+def matvec_bytes(in_use, columns, W):
+    return in_use * 6 * W + columns * (13 * W + 4 + 12 + 4)
+
+
+def update_bytes(in_use, columns, W):
+    F = 2 if W == 4 else 8
+    return in_use * (4 * W + 2 * F) + columns * (8 if W == 4 else 4)
+
+
 def measured_traffic(name):
     """HBM bytes per launch of a kernel on this workload, from the rocprofv3 FETCH_SIZE / WRITE_SIZE
     summary kept in profiles/<name>.txt (line "traffic_bytes_per_launch: N"), or None if absent."""
@@ -264,8 +286,15 @@ def main():
     # the first iteration of each inner solve (one per refinement step) has no pending x update
     first_frac = mx["stats"][-1]["outer_iters"] / max(mx["stats"][-1]["inner_iters"], 1)
     table = mx["stats"][-1].get("zw_table", 0) == 1
-    kern_bytes = int(bwd_bytes(cells, columns, 4, table) - first_frac * 8 * cells)
-    mv_bytes = MATVEC_BYTES[4] * cells
+    streaming = args.tile_rows == 0 and args.buffer_addressing == 0 and args.zw_table == 0
+    # the cells that the kernels work on, and the bytes of a launch: by word size
+    work = {W: cells_in_use(g, W) if streaming else cells for W in (4, 8)}
+    mv_name, up_name = ("k_matvec", "k_update") if streaming else ("k_bwd", "k_fwd")
+    mv_kernel = {W: matvec_bytes(work[W], columns, W) if streaming else bwd_bytes(cells, columns, W, t)
+                 for W, t in ((4, table), (8, f64["stats"][-1].get("zw_table", 0) == 1))}
+    up_kernel = {W: (update_bytes if streaming else fwd_bytes)(work[W], columns, W) for W in (4, 8)}
+    kern_bytes = int(mv_kernel[4] - first_frac * (12 if streaming else 8) * work[4])
+    mv_bytes = MATVEC_BYTES[4] * work[4]
     achieved = mv_bytes / (mv_avg_ms * 1e-3) / 1e9
     prof64 = f64["prof"]
     mv64_ms = prof64["matvec_ms"] / max(prof64["matvec_launches"], 1)
@@ -303,25 +332,26 @@ def main():
         "latency_ms_p99": round(pct(mx["lat"], 99), 3),
         "latency_ms_p50_fp64": round(pct(f64["lat"], 50), 3),
         "latency_ms_p99_fp64": round(pct(f64["lat"], 99), 3),
-        "roofline": {"bound": "hbm", "kernel": "k_bwd<float> (7-point matvec + back substitution + p update + p.q)",
+        "roofline": {"bound": "hbm", "kernel": mv_name + ("<float> (7-point matvec + p update + p.q)" if streaming else
+                                                  "<float> (7-point matvec + back substitution + p update + p.q)"),
                      "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": (measured_traffic("traffic_k_bwd_f32_regional_1024x768x60")
+                     "traffic": (measured_traffic(f"traffic_{mv_name}_f32_regional_1024x768x60")
                                  if args.buffer_addressing == 0 else None),
                      "bytes_per_launch": mv_bytes, "bytes_per_cell": MATVEC_BYTES[4],
-                     "bytes_note": "the bare matvec y = A x: 7 coefficients + x + y per cell (FP32)",
-                     "kernel_bytes_per_launch": kern_bytes, "kernel_GBps": round(kern_bytes / (mv_avg_ms * 1e-3) / 1e9, 1),
+                     "bytes_note": "the bare matvec y = A x: 7 coefficients + x + y per cell (FP32)"
+                                   + (" of the levels in use" if streaming else ""),
+                     "cells_in_use": work[4], "kernel_bytes_per_launch": kern_bytes, "kernel_GBps": round(kern_bytes / (mv_avg_ms * 1e-3) / 1e9, 1),
                      "zw_table": int(table), "buffer_addressing": mx["stats"][-1].get("buffer_addressing", 0),
                      "avg_launch_ms": round(mv_avg_ms, 5), "launches": prof["matvec_launches"]},
         "other_kernels": {
-            "k_fwd<float>": {"avg_launch_ms": round(up_avg_ms, 5), "bytes_per_cell": 20, "bytes_per_column": 4,
-                             "GBps": round(fwd_bytes(cells, columns, 4) / (up_avg_ms * 1e-3) / 1e9, 1)},
-            "k_bwd<double>": {"avg_launch_ms": round(mv64_ms, 5), "matvec_bytes_per_cell": MATVEC_BYTES[8],
-                              "matvec_GBps": round(MATVEC_BYTES[8] * cells / (mv64_ms * 1e-3) / 1e9, 1),
-                              "kernel_GBps": round(bwd_bytes(cells, columns, 8, f64["stats"][-1].get("zw_table", 0) == 1)
-                                                   / (mv64_ms * 1e-3) / 1e9, 1)},
-            "k_fwd<double>": {"avg_launch_ms": round(up64_ms, 5), "bytes_per_cell": 48,
-                              "GBps": round(fwd_bytes(cells, columns, 8) / (up64_ms * 1e-3) / 1e9, 1)},
+            up_name + "<float>": {"avg_launch_ms": round(up_avg_ms, 5), "bytes_per_cell": 20,
+                                  "GBps": round(up_kernel[4] / (up_avg_ms * 1e-3) / 1e9, 1)},
+            mv_name + "<double>": {"avg_launch_ms": round(mv64_ms, 5), "matvec_bytes_per_cell": MATVEC_BYTES[8],
+                                   "matvec_GBps": round(MATVEC_BYTES[8] * work[8] / (mv64_ms * 1e-3) / 1e9, 1),
+                                   "kernel_GBps": round(mv_kernel[8] / (mv64_ms * 1e-3) / 1e9, 1)},
+            up_name + "<double>": {"avg_launch_ms": round(up64_ms, 5), "bytes_per_cell": 48,
+                                   "GBps": round(up_kernel[8] / (up64_ms * 1e-3) / 1e9, 1)},
         },
         "copy_probe_GBps": round(abi.copy_probe(1 << 30, 20), 1),
         "device": device_state(),
@@ -429,7 +459,7 @@ def bench_batch(args):
     mv_gbs = mx["mv_bytes"] / (prof["matvec_ms"] * 1e-3) / 1e9
     # the counted traffic of the 64-system mixed batch (rocprofv3 summary in profiles/)
     traffic = None
-    if "mixed" in out and args.nsys == 64 and args.scale == 1.0 and args.tile_rows in (0, 12) and args.zw_table == 0 \
+    if "mixed" in out and args.nsys == 64 and args.scale == 1.0 and args.tile_rows == 12 and args.zw_table == 0 \
             and args.buffer_addressing == 0:
         traffic = measured_traffic("traffic_k_bwd_f32_batch_64systems")
     line = {
@@ -449,10 +479,11 @@ def bench_batch(args):
         "tile_rows_mixed": mx["heights"], "tile_rows_fp64": f64["heights"] if f64 else None,
         "latency_ms_p50": round(pct(mx["lat"], 50), 3), "latency_ms_p99": round(pct(mx["lat"], 99), 3),
         "device": device_state(),
-        "roofline": {"bound": "hbm", "kernel": "k_bwd<float> (batched)", "achieved": round(mv_gbs, 1),
+        "roofline": {"bound": "hbm", "kernel": "inner matvec, FP32 (batched)", "achieved": round(mv_gbs, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(mv_gbs / HBM_PEAK_GBS, 4),
                      "traffic": traffic, "bytes_per_launch": MATVEC_BYTES[4] * cells,
-                     "note": "the bare matvec bytes (36 B per cell, FP32) per active cell-iteration over the "
+                     "note": "the bare matvec bytes (36 B per cell of the box, dry ones that the kernels skip too, FP32) per "
+                             "active cell-iteration over the "
                              "summed matvec launch time; bytes_per_launch and traffic (HBM bytes counted by "
                              "FETCH_SIZE/WRITE_SIZE) are those of one launch in which every system iterates"},
         "cpu_baseline": None,
@@ -621,7 +652,7 @@ def bench_serve(args):
         "cell_solves_per_s": round(nsteps * burst["cells"] / burst["wall"], 1),
         "mean_inner_iters_per_step": round(burst["inner"] / solves, 2),
         "max_rel_res": max(burst["rel"], steady["rel"] if steady else 0.0),
-        "roofline": {"bound": "hbm", "kernel": "k_bwd<float> over the whole burst", "achieved": round(mv_gbs, 1),
+        "roofline": {"bound": "hbm", "kernel": "inner matvec, FP32, over the whole burst", "achieved": round(mv_gbs, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(mv_gbs / HBM_PEAK_GBS, 4), "traffic": None,
                      "note": "the inner matvec's bytes (36 B per cell, FP32) of every inner iteration served, over "
                              "the burst's wall time (admission, cohort set-up, the other kernels and idle lanes "

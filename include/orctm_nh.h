@@ -92,8 +92,10 @@ typedef struct orctm_nh_options {
   int32_t check_every;  /* inner iterations per device-side chunk between host polls (default 16) */
   int32_t device;       /* HIP device ordinal (default 0) */
   int32_t profile;      /* 1: time the inner kernels with HIP events (orctm_nh_profile_read); default 0 */
-  int32_t tile_rows;    /* rows (j) per tile of the inner-iteration kernels: 0 (default) = tuned per size
-                           class at create / batch create; 4, 8 or 12 = fixed. Results are the same bits
+  int32_t tile_rows;    /* rows (j) per tile of the inner-iteration kernels: 0 (default) = chosen by size:
+                           launches of few columns run on blocks of columns and those of many, up to 64
+                           levels, on streaming kernels of 4 rows; the rest on tiled kernels tuned per size class at create / batch create.
+                           4, 8 or 12 = the tiled kernels at that height. Results are the same bits
                            for every choice (block sums are formed over fixed 4-row groups). Tuned picks
                            persist per device (arch/CU count), precision and size class in a JSON file:
                            $ORCTM_NH_TUNE_FILE (set but empty: none), else
@@ -105,8 +107,9 @@ typedef struct orctm_nh_options {
                            the shipped Makefile builds (-DZZCG2D4NONHY). */
   int32_t zw_table;     /* where the iteration kernels read ZW/ZP (stats.zw_table reports the choice):
                            0 (default) = from the per-level table and per-column window when they
-                           reproduce every column (checked at create) and the solve launches cover at
-                           least 2^20 cells (one system, or a batch in total), else the per-cell planes;
+                           reproduce every column (checked at create) and the solve launches run the
+                           streaming kernels or cover at least 2^20 cells (one system, or a batch in
+                           total), else the per-cell planes;
                            1 = the table whenever it reproduces every column; -1 = always the planes.
                            Results are the same bits for every choice. */
   int32_t buffer_addressing; /* how the matvec kernel addresses memory (stats.buffer_addressing reports the
@@ -298,8 +301,10 @@ typedef struct orctm_nh_sor_grid {
   int32_t cyclic_x, cyclic_y;  /* ICYCLI_X, ICYCLI_Y */
   int32_t iterations;          /* red-black sweeps per solve (250 in troneu.f90:103) */
   int32_t device;              /* HIP device ordinal */
-  int32_t half_sweeps;         /* half-sweeps per blocked device launch: 0 = the fastest of 4, 6, 7, 8, 12, timed at
-                                  creation; or one of them. Results are bit-identical for every choice */
+  int32_t half_sweeps;         /* half-sweeps per blocked device launch: 0 = all in one launch where one block
+                                  holds the surface (sor_info then reports 12 and 1 launch), else the fastest
+                                  of 4, 6, 7, 8, 12, timed at creation; or one of them. Results are
+                                  bit-identical for every choice */
   int32_t reserved;            /* 0 */
   const double* dlxp;          /* DLXP(IE,JE) */
   const double* dlyp;          /* DLYP(IE,JE) */

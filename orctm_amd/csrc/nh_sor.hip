@@ -9,6 +9,7 @@
 // half-sweeps run temporally blocked (nh_sor_tb.h: several half-sweeps per launch, staged in LDS, the
 // cyclic halo read through a periodic index map), ending with one exchange. Within a colour every
 // update reads only values from before the half-sweep, so every schedule gives the reference's bits.
+// A surface that one block holds runs every half-sweep in one launch (k_sor_one).
 // The whole sequence is captured once into a hipGraph and replayed per call; the half-sweeps per launch
 // are chosen by timing the compiled depths at creation. FP64 throughout, expressions left to right as
 // the Fortran source writes them (no contraction).
