@@ -213,7 +213,7 @@ hipError_t opalloc(orctm_nh_t* h, void** p, size_t bytes) {
   return e == hipSuccess ? hipStreamSynchronize(h->stream) : e;
 }
 
-// Per-handle state: right-hand side, solution, inner work vectors, block partials, ||b||.
+// Per-handle state: right-hand side, solution, inner work vectors and their levels in use, block partials, ||b||.
 int alloc_state(orctm_nh_t* h) {
   const size_t NP = (size_t)h->plane * h->nz;
   const size_t es = h->fp32 ? sizeof(float) : sizeof(double);
@@ -234,6 +234,7 @@ int alloc_state(orctm_nh_t* h) {
   SALLOC(pa, NP * es, void*);
   SALLOC(pb, NP * es, void*);
   SALLOC(q, NP * es, void*);
+  SALLOC(use, (size_t)h->plane * sizeof(int), int*);
   SALLOC(partials, 2 * (size_t)s.nslots * sizeof(double), double*);
   // sums of nh_small.hip: per 64-column row, or per column where a block may take fewer
   const size_t rows64 = (size_t)s.tiles_x * s.ny;
@@ -1161,7 +1162,6 @@ int create_device(orctm_nh_t* h, const orctm_nh_grid_t* g) {
   ALLOC(tp, (size_t)h->nz * sizeof(double), const double*);
   ALLOC(xk, (size_t)h->plane * sizeof(int), const int*);
   ALLOC(xf, 3 * (size_t)h->plane * sizeof(uint32_t), const uint32_t*);
-  ALLOC(use, (size_t)h->plane * sizeof(int), int*);
   ALLOC(xw, 3 * (size_t)h->plane * sizeof(double), const double*);
   ALLOC(xp, 3 * (size_t)h->plane * sizeof(double), const double*);
   if (h->fp32) {

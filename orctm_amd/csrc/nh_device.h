@@ -83,9 +83,6 @@ struct Sys {
   // (periodic or not on the domain edge); with `tab` set the kernels derive each cell's flag bits from
   // them instead of reading the flag plane (checked bit for bit against it at create)
   const uint32_t* xf;
-  // with `tab`: per column, the levels that the inner solve at hand works on (k_residual): the most wet levels
-  // and the deepest nonzero of r of the 16 columns around it. The other levels of r, x, z, p and q are 0 or unused.
-  int* use;
   const void* invD;     // line preconditioner 1/D_k: FP64, or fp16 bits scaled by dscale (FP32)
   const void* L;        // line preconditioner l_k: FP64, or fp16 bits (FP32)
   const float* dscale;  // FP32 only: per-column power of two that multiplies the stored invD
@@ -97,11 +94,15 @@ struct Sys {
   void* pa;             // search direction, buffer A
   void* pb;             // search direction, buffer B
   void* q;              // C p
+  // with `tab`: per column, the levels that the inner solve at hand works on (k_residual): the most wet levels
+  // and the deepest nonzero of r of the kUseBytes of a row around it. The other levels of r, x, z, p and q are 0 or
+  // unused. It follows r, so it belongs to the state: handles that share an operator each have their own.
+  int* use;
   double* partials;     // 2*nslots partial sums (summed by the reduction kernel in slot order)
   Outer* outer;
   void* inner;          // Inner<T>*
   void* inner2;         // second copy of the inner state (launches of few columns, nh_small.hip)
-  void* rowsum;         // 2 x 2 x tiles_x*ny sums over the 64-column rows (the same launches)
+  void* rowsum;         // their sums: 2 x 2 for each 64-column row, or for each column of few (kSmallColumns)
   double* nbp;          // ||b||_2 of the resident right-hand side (written by the rhs kernel)
   const double* smaxp;  // max S of the system (written by the assembly)
   double rtol, rtol_inner;

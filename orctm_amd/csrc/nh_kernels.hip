@@ -174,7 +174,6 @@ __global__ __launch_bounds__(NT) void k_zflags(const Sys* __restrict__ systems, 
   xf[col] = w[0];
   xf[P + col] = w[1];
   xf[2 * P + col] = w[2];
-  s.use[col] = (int)(w[0] & 0xffffu);  // for the timing of tile heights, before the first residual
   gptr<const uint16_t> flg = G<const uint16_t>(s.flg);
   bool diff = false;
   for (int K = 1; K <= f.KE; ++K) diff = diff || flg[(size_t)(K - 1) * P + col] != flags_from_words(K, f.KE, w);
