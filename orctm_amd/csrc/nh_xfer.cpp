@@ -26,12 +26,11 @@ Stage g_stage[kStages];
 std::mutex g_count_mu;
 int g_handles = 0;
 
-bool made(const Stage& s, int workers, int device) {
-  if (s.device != device) return false;
-  for (int w = 0; w < workers; ++w)
-    for (int q = 0; q < 2; ++q)
-      if (!s.buf[w][q] || !s.ev[w][q]) return false;
-  return true;
+// Workers whose buffers and events are there.
+int made(const Stage& s, int device) {
+  int w = 0;
+  while (s.device == device && w < kXferWorkers && s.buf[w][0] && s.buf[w][1] && s.ev[w][0] && s.ev[w][1]) ++w;
+  return w;
 }
 
 void drop(Stage& s) {
@@ -45,7 +44,8 @@ void drop(Stage& s) {
   s.device = -1;
 }
 
-hipError_t make(Stage& s, int workers, int device) {
+// Buffers and events for `workers`, or for as many as there is memory to pin.
+void make(Stage& s, int workers, int device) {
   if (s.device != device) drop(s);
   s.device = device;
   for (int w = 0; w < workers; ++w)
@@ -57,9 +57,11 @@ hipError_t make(Stage& s, int workers, int device) {
         s.buf[w][q] = static_cast<char*>(p);
       }
       if (e == hipSuccess && !s.ev[w][q]) e = hipEventCreateWithFlags(&s.ev[w][q], hipEventDisableTiming);
-      if (e != hipSuccess) return e;
+      if (e != hipSuccess) {
+        (void)hipGetLastError();  // or the next launch's check reports it
+        return;
+      }
     }
-  return hipSuccess;
 }
 
 struct Chunk {
@@ -143,34 +145,55 @@ hipError_t work(Stage& s, int w, const Plan& plan, std::atomic<size_t>& next, bo
   return err;
 }
 
+// The pieces through the runtime's own copies: flat ones queued, rows a plane at a time.
+hipError_t direct(hipStream_t st, const XferPiece* p, int n, bool to_host) {
+  hipError_t e = hipSuccess;
+  for (int q = 0; q < n && e == hipSuccess; ++q) {
+    if (!p[q].flat()) continue;
+    e = to_host ? hipMemcpyAsync(p[q].host, p[q].dev, p[q].bytes(), hipMemcpyDeviceToHost, st)
+                : hipMemcpyAsync(p[q].dev, p[q].host, p[q].bytes(), hipMemcpyHostToDevice, st);
+  }
+  const hipError_t es = hipStreamSynchronize(st);
+  if (e == hipSuccess) e = es;
+  for (int q = 0; q < n; ++q) {
+    if (p[q].flat() || !p[q].bytes()) continue;
+    std::lock_guard<std::recursive_mutex> dev(device_lock());
+    const size_t w = sizeof(double), pitch = p[q].dev_pitch ? p[q].dev_pitch * w : p[q].row_bytes,
+                 plane = p[q].dev_pitch ? p[q].dev_plane * w : p[q].row_bytes * p[q].rows;
+    for (size_t k = 0; k < p[q].planes && e == hipSuccess; ++k) {
+      char *h = p[q].host + k * p[q].plane_stride, *d = p[q].dev + k * plane;
+      e = to_host ? hipMemcpy2D(h, p[q].row_stride, d, pitch, p[q].row_bytes, p[q].rows, hipMemcpyDeviceToHost)
+                  : hipMemcpy2D(d, pitch, h, p[q].row_stride, p[q].row_bytes, p[q].rows, hipMemcpyHostToDevice);
+    }
+  }
+  return e;
+}
+
 hipError_t transfer(int device, hipStream_t st, const XferPiece* p, int n, bool to_host) {
   if (n < 0 || n > kXferPieces) return hipErrorInvalidValue;
   size_t bytes = 0;
   bool flat = true;
   for (int q = 0; q < n; ++q) {
     bytes += p[q].bytes();
-    flat = flat && p[q].rows * p[q].planes == 1 && !p[q].dev_pitch;
+    flat = flat && p[q].flat();
   }
-  if (flat && bytes < (to_host ? kXferDirectHost : kXferDirectDevice)) {
-    hipError_t e = hipSuccess;
-    for (int q = 0; q < n && e == hipSuccess; ++q)
-      e = to_host ? hipMemcpyAsync(p[q].host, p[q].dev, p[q].bytes(), hipMemcpyDeviceToHost, st)
-                  : hipMemcpyAsync(p[q].dev, p[q].host, p[q].bytes(), hipMemcpyHostToDevice, st);
-    const hipError_t es = hipStreamSynchronize(st);
-    return e != hipSuccess ? e : es;
-  }
+  if (flat && bytes < (to_host ? kXferDirectHost : kXferDirectDevice)) return direct(st, p, n, to_host);
   const size_t part = (bytes / 12 + 7) / 8 * 8;
   const Plan plan(p, n, to_host ? std::min(std::max(part, kXferChunk / 8), kXferChunk) : kXferChunk);
   if (plan.chunks() == 0) return hipSuccess;
-  const int want = bytes >= kXferThreaded ? (int)std::min<size_t>(kXferWorkers, plan.chunks()) : 1;
+  int want = bytes >= kXferThreaded ? (int)std::min<size_t>(kXferWorkers, plan.chunks()) : 1;
   Stage& s = g_stage[(unsigned)device % kStages];
   std::unique_lock<std::mutex> lk(s.mu);
-  while (!made(s, want, device)) {  // allocates: not while another thread captures a graph
+  if (made(s, device) < want) {  // allocates: not while another thread captures a graph
     lk.unlock();
     std::lock_guard<std::recursive_mutex> dev(device_lock());
     lk.lock();
-    const hipError_t e = make(s, want, device);
-    if (e != hipSuccess) return e;
+    make(s, want, device);
+  }
+  want = std::min(want, made(s, device));
+  if (want == 0) {  // no memory to pin
+    lk.unlock();
+    return direct(st, p, n, to_host);
   }
   std::atomic<size_t> next{0};
   hipError_t got[kXferWorkers] = {};

@@ -13,7 +13,8 @@
 // Contiguous transfers below kXferDirectDevice and kXferDirectHost go to the runtime as they are: its own
 // staging is as fast there (128x128x30 to the device: 0.16 ms).
 // The pinned buffers (kXferWorkers * 2 chunks, 32 MiB) and their events belong to the device, one set for
-// each that transfers, held by one transfer at a time; they are freed with the process's last handle.
+// each that transfers, held by one transfer at a time; they are freed with the process's last handle. Where no
+// memory can be pinned, a transfer works with as many workers as have their buffers, or through the runtime.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -37,6 +38,7 @@ struct XferPiece {
   char* dev = nullptr;
   size_t dev_pitch = 0, dev_plane = 0;
   size_t bytes() const { return row_bytes * rows * planes; }
+  bool flat() const { return rows * planes == 1 && !dev_pitch; }
 };
 
 XferPiece xfer_flat(void* dev, const void* host, size_t bytes);

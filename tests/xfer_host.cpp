@@ -1,0 +1,139 @@
+// The transfers of orctm_amd/csrc/nh_xfer.cpp on the host, over a runtime of this file's own in which device memory
+// is host memory and a copy is done when it is queued. Each check is an argument; prints OK.
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+
+#include <atomic>
+#include <future>
+#include <set>
+#include <vector>
+
+#include "../orctm_amd/csrc/nh_xfer.cpp"
+
+static std::atomic<long> g_pins{0}, g_pin_limit{1 << 20}, g_copies{0};
+static thread_local hipError_t g_last = hipSuccess;
+
+std::recursive_mutex& onh::device_lock() {
+  static std::recursive_mutex m;
+  return m;
+}
+
+extern "C" {
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  if (g_pins >= g_pin_limit) {
+    *p = nullptr;
+    return g_last = hipErrorOutOfMemory;
+  }
+  ++g_pins;
+  *p = malloc(n);
+  return hipSuccess;
+}
+hipError_t hipHostFree(void* p) {
+  --g_pins;
+  free(p);
+  return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+  *e = reinterpret_cast<hipEvent_t>(malloc(1));
+  return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t e) {
+  free(e);
+  return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetLastError() {
+  const hipError_t e = g_last;
+  g_last = hipSuccess;
+  return e;
+}
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+  ++g_copies;
+  memcpy(d, s, n);
+  return hipSuccess;
+}
+hipError_t hipMemcpy2D(void* d, size_t dp, const void* s, size_t sp, size_t w, size_t h, hipMemcpyKind) {
+  ++g_copies;
+  for (size_t r = 0; r < h; ++r) memcpy((char*)d + r * dp, (const char*)s + r * sp, w);
+  return hipSuccess;
+}
+}
+
+hipError_t onh::launch_pack(hipStream_t, const double* src, size_t pitch, size_t plane, size_t nx, size_t ny, size_t first,
+                            size_t n, double* out) {
+  for (size_t t = 0; t < n; ++t) {
+    const size_t e = first + t, row = e / nx;
+    out[t] = src[row / ny * plane + row % ny * pitch + e % nx];
+  }
+  return hipSuccess;
+}
+
+using namespace onh;
+
+static void need(bool ok, const char* what) {
+  if (ok) return;
+  printf("failed: %s\n", what);
+  exit(1);
+}
+
+static std::vector<double> numbers(size_t n, double at) {
+  std::vector<double> v(n);
+  for (size_t i = 0; i < n; ++i) v[i] = at + (double)i;
+  return v;
+}
+
+// An interior of IE x JE x KE to the host and two arrays each way, compared with loops.
+static void round_trip(int IE, int JE, int KE, size_t flat, hipStream_t st = nullptr) {
+  const size_t pitch = (size_t)(IE - 2 + 31) / 32 * 32, plane = pitch * (size_t)(JE - 2);
+  const std::vector<double> dev = numbers(plane * KE, 0.5);
+  std::vector<double> host = numbers((size_t)IE * JE * KE, -1e9), want = host;
+  for (int k = 0; k < KE; ++k)
+    for (int j = 0; j < JE - 2; ++j)
+      for (int i = 0; i < IE - 2; ++i)
+        want[(size_t)(i + 1) + (size_t)IE * (j + 1 + (size_t)JE * k)] = dev[(size_t)i + pitch * j + plane * k];
+  const XferPiece p = xfer_interior((void*)dev.data(), host.data(), IE, JE, KE, pitch, plane);
+  need(xfer_to_host(0, st, &p, 1) == hipSuccess && host == want, "interior to the host");
+  for (const bool down : {false, true}) {
+    const std::vector<double> a = numbers(flat, 1.0), b = numbers(flat / 3 + 1, 7.0);
+    std::vector<double> x(a.size()), y(b.size());
+    XferPiece two[2];
+    if (down) {
+      two[0] = xfer_flat((void*)a.data(), x.data(), a.size() * 8);
+      two[1] = xfer_flat((void*)b.data(), y.data(), b.size() * 8);
+    } else {
+      two[0] = xfer_flat(x.data(), a.data(), a.size() * 8);
+      two[1] = xfer_flat(y.data(), b.data(), b.size() * 8);
+    }
+    need((down ? xfer_to_host(0, st, two, 2) : xfer_to_device(0, st, two, 2)) == hipSuccess && x == a && y == b,
+         down ? "arrays to the host" : "arrays to the device");
+  }
+}
+
+static const struct {
+  int IE, JE, KE;
+  size_t flat;
+} kSizes[] = {{3, 3, 1, 1}, {99, 43, 5, 1000}, {130, 130, 32, 600000}, {131, 129, 40, 2100000}, {333, 301, 41, 5000003}};
+
+// As much memory as there is to pin, from none to all of it.
+static void no_memory_to_pin() {
+  for (long limit = 0; limit <= 2 * kXferWorkers + 1; ++limit) {
+    xfer_retain();
+    g_pin_limit = limit;
+    for (const auto& s : kSizes) round_trip(s.IE, s.JE, s.KE, s.flat);
+    need(g_last == hipSuccess, "no error is left behind");
+    xfer_release();
+    need(g_pins == 0, "the chunks are given back");
+  }
+}
+
+int main(int argc, char** argv) {
+  const char* what = argc > 1 ? argv[1] : "";
+  if (!strcmp(what, "pin")) no_memory_to_pin();
+  else need(false, "an unknown check");
+  printf("OK\n");
+  return 0;
+}
