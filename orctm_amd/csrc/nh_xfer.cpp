@@ -6,7 +6,6 @@
 #include <algorithm>
 #include <atomic>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 #include "nh_lock.h"
@@ -204,8 +203,8 @@ hipError_t transfer(int device, hipStream_t st, const XferPiece* p, int n, bool 
         const hipError_t e = hipSetDevice(device);
         got[w] = e == hipSuccess ? work(s, w, plan, next, to_host, st) : e;
       });
-    } catch (const std::system_error&) {
-      break;  // no thread to be had: the others take its share
+    } catch (...) {
+      break;  // no thread or no memory for one to be had: the others take its share
     }
   }
   got[0] = work(s, 0, plan, next, to_host, st);

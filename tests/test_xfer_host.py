@@ -1,7 +1,8 @@
 """The transfers between the caller's arrays and the device (orctm_amd/csrc/nh_xfer.cpp), compiled for the host over a
 runtime of the harness's own (tests/xfer_host.cpp): what arrives where, and what happens when
 
-* only some of the chunks, or none, can be pinned (``pin``): fewer workers, or the runtime's own copies.
+* only some of the chunks, or none, can be pinned (``pin``): fewer workers, or the runtime's own copies;
+* no thread can be started (``threads``): the caller does all the work.
 """
 import os
 import shutil
@@ -23,7 +24,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["pin"])
+@pytest.mark.parametrize("check", ["pin", "threads"])
 def test_transfer(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.strip() == "OK", r.stdout + r.stderr

@@ -6,13 +6,23 @@
 
 #include <atomic>
 #include <future>
+#include <new>
 #include <set>
 #include <vector>
 
 #include "../orctm_amd/csrc/nh_xfer.cpp"
 
 static std::atomic<long> g_pins{0}, g_pin_limit{1 << 20}, g_copies{0};
+static std::atomic<bool> g_no_new{false};
 static thread_local hipError_t g_last = hipSuccess;
+
+void* operator new(size_t n) {
+  if (g_no_new) throw std::bad_alloc();
+  if (void* p = malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
 
 std::recursive_mutex& onh::device_lock() {
   static std::recursive_mutex m;
@@ -130,9 +140,25 @@ static void no_memory_to_pin() {
   }
 }
 
+// No thread to be had: nothing can be allocated while the transfer runs.
+static void no_threads() {
+  xfer_retain();
+  round_trip(333, 301, 41, 5000003);
+  const size_t n = 5000003;
+  const std::vector<double> a = numbers(n, 3.0);
+  std::vector<double> x(n);
+  const XferPiece p = xfer_flat(x.data(), a.data(), n * 8);
+  g_no_new = true;
+  const hipError_t e = xfer_to_device(0, nullptr, &p, 1);
+  g_no_new = false;
+  need(e == hipSuccess && x == a, "one worker alone");
+  xfer_release();
+}
+
 int main(int argc, char** argv) {
   const char* what = argc > 1 ? argv[1] : "";
   if (!strcmp(what, "pin")) no_memory_to_pin();
+  else if (!strcmp(what, "threads")) no_threads();
   else need(false, "an unknown check");
   printf("OK\n");
   return 0;
