@@ -11,7 +11,10 @@
 // ones lose more to the copies' own overhead than the overlap gains (128x128x30: 0.20 ms in one chunk,
 // 0.28 in 12).
 // Contiguous transfers below kXferDirectDevice and kXferDirectHost go to the runtime as they are: its own
-// staging is as fast there (128x128x30 to the device: 0.16 ms).
+// staging is as fast there (128x128x30 to the device: 0.16 ms). So do arrays that the runtime holds already (pinned by
+// the caller): the device reads and writes them itself (1024x768x60 to the device: 6.8 ms, 8.4 through the chunks;
+// 256x256x33: 0.35, 0.53), rows of an interior from kXferHeldRows on (to the host 7.1 ms, 7.5 through the chunks;
+// below, the copy commands of the levels cost more than the chunks: 400x300x40 0.98 ms, 0.88; 128x128x30 0.29, 0.17).
 // The pinned buffers (kXferWorkers * 2 chunks, 32 MiB) and their events belong to the device, one set for
 // each that transfers, held by one transfer at a time; they are freed with the process's last handle. Where no
 // memory can be pinned, a transfer works with as many workers as have their buffers, or through the runtime.
@@ -27,6 +30,7 @@ constexpr int kXferWorkers = 4;
 constexpr size_t kXferThreaded = size_t(4) << 20;
 constexpr size_t kXferDirectDevice = size_t(16) << 20;
 constexpr size_t kXferDirectHost = size_t(1) << 20;
+constexpr size_t kXferHeldRows = size_t(64) << 20;
 
 // One piece: on the host `planes` planes of `rows` rows of `row_bytes` bytes; on the device the same bytes in
 // that order, contiguous, or (dev_pitch != 0, reading from the device only) doubles at

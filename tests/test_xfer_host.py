@@ -2,7 +2,8 @@
 runtime of the harness's own (tests/xfer_host.cpp): what arrives where, and what happens when
 
 * only some of the chunks, or none, can be pinned (``pin``): fewer workers, or the runtime's own copies;
-* no thread can be started (``threads``): the caller does all the work.
+* no thread can be started (``threads``): the caller does all the work;
+* the runtime holds the caller's arrays already (``held``): its copies take them as they are.
 """
 import os
 import shutil
@@ -24,7 +25,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["pin", "threads"])
+@pytest.mark.parametrize("check", ["pin", "threads", "held"])
 def test_transfer(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.strip() == "OK", r.stdout + r.stderr

@@ -15,6 +15,7 @@
 static std::atomic<long> g_pins{0}, g_pin_limit{1 << 20}, g_copies{0};
 static std::atomic<bool> g_no_new{false};
 static thread_local hipError_t g_last = hipSuccess;
+static std::set<const void*> g_held;  // arrays pinned by the caller
 
 void* operator new(size_t n) {
   if (g_no_new) throw std::bad_alloc();
@@ -60,6 +61,14 @@ hipError_t hipGetLastError() {
   const hipError_t e = g_last;
   g_last = hipSuccess;
   return e;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
+  for (const void* h : g_held)
+    if (p >= h && p < (const char*)h + (size_t(1) << 30)) {
+      a->type = hipMemoryTypeHost;
+      return hipSuccess;
+    }
+  return g_last = hipErrorInvalidValue;
 }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
   ++g_copies;
@@ -155,10 +164,42 @@ static void no_threads() {
   xfer_release();
 }
 
+// Arrays that the caller pinned are copied by the runtime, in one piece each; an interior of fewer bytes than
+// kXferHeldRows and one array of two that is pinned go through the chunks.
+static void held_by_the_runtime() {
+  xfer_retain();
+  const size_t n = 5000003, IE = 402, JE = 302, KE = 100, pitch = 416, plane = pitch * 300;
+  std::vector<double> dev = numbers(n, 3.0), box = numbers(plane * KE, 0.0);
+  char* mem = (char*)calloc(size_t(1) << 30, 1);
+  double* host = (double*)mem;
+  g_held.insert(mem);
+  XferPiece two[2] = {xfer_flat(dev.data(), host, n * 8), xfer_flat(dev.data(), host + n, n * 8)};
+  g_copies = 0;
+  need(xfer_to_host(0, nullptr, two, 2) == hipSuccess && g_copies == 2 && g_pins == 0, "pinned arrays to the host");
+  need(!memcmp(host, dev.data(), n * 8) && !memcmp(host + n, dev.data(), n * 8), "their values");
+  need(xfer_to_device(0, nullptr, two, 2) == hipSuccess && g_copies == 4 && g_pins == 0, "pinned arrays to the device");
+  XferPiece in = xfer_interior(box.data(), host, IE, JE, KE, pitch, plane);
+  need(in.bytes() >= kXferHeldRows && xfer_to_host(0, nullptr, &in, 1) == hipSuccess && g_pins == 0, "pinned rows");
+  for (size_t k = 0; k < KE; ++k)
+    for (size_t j = 0; j < JE - 2; ++j)
+      need(!memcmp(host + 1 + IE * (j + 1 + JE * k), box.data() + plane * k + pitch * j, (IE - 2) * 8), "their values");
+  in = xfer_interior(box.data(), host, IE, JE, 10, pitch, plane);
+  need(xfer_to_host(0, nullptr, &in, 1) == hipSuccess && g_pins > 0, "few pinned rows");
+  std::vector<double> other(n);
+  two[0] = xfer_flat(dev.data(), other.data(), n * 8);
+  g_copies = 0;
+  need(xfer_to_host(0, nullptr, two, 2) == hipSuccess && g_copies > 2 && other == dev, "one of two pinned");
+  need(g_last == hipSuccess, "no error is left behind");
+  xfer_release();
+  g_held.clear();
+  free(mem);
+}
+
 int main(int argc, char** argv) {
   const char* what = argc > 1 ? argv[1] : "";
   if (!strcmp(what, "pin")) no_memory_to_pin();
   else if (!strcmp(what, "threads")) no_threads();
+  else if (!strcmp(what, "held")) held_by_the_runtime();
   else need(false, "an unknown check");
   printf("OK\n");
   return 0;
