@@ -21,7 +21,7 @@ struct Stage {
 };
 
 constexpr int kStages = 16;  // device ordinals beyond share them
-Stage g_stage[kStages];
+Stage g_stage[2][kStages];   // to the device, to the host
 std::mutex g_count_mu;
 int g_handles = 0;
 
@@ -192,7 +192,15 @@ hipError_t transfer(int device, hipStream_t st, const XferPiece* p, int n, bool 
   const Plan plan(p, n, to_host ? std::min(std::max(part, kXferChunk / 8), kXferChunk) : kXferChunk);
   if (plan.chunks() == 0) return hipSuccess;
   int want = bytes >= kXferThreaded ? (int)std::min<size_t>(kXferWorkers, plan.chunks()) : 1;
-  Stage& s = g_stage[(unsigned)device % kStages];
+  // kernels that the transfer follows end before it holds the stage: it holds others up for its copies' time alone
+  // (asked first: a wait puts a marker of its own on the stream, 20 us of a 128x128x30 interior's 170)
+  hipError_t es = hipStreamQuery(st);
+  if (es == hipErrorNotReady) {
+    (void)hipGetLastError();
+    es = hipStreamSynchronize(st);
+  }
+  if (es != hipSuccess) return es;
+  Stage& s = g_stage[to_host][(unsigned)device % kStages];
   std::unique_lock<std::mutex> lk(s.mu);
   if (made(s, device) < want) {  // allocates: not while another thread captures a graph
     lk.unlock();
@@ -269,10 +277,11 @@ void xfer_release() {
   std::lock_guard<std::recursive_mutex> dev(device_lock());
   std::lock_guard<std::mutex> lk(g_count_mu);
   if (--g_handles > 0) return;
-  for (Stage& s : g_stage) {
-    std::lock_guard<std::mutex> ls(s.mu);
-    if (s.device >= 0) drop(s);
-  }
+  for (auto& way : g_stage)
+    for (Stage& s : way) {
+      std::lock_guard<std::mutex> ls(s.mu);
+      if (s.device >= 0) drop(s);
+    }
 }
 
 }  // namespace onh

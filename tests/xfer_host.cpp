@@ -1,11 +1,15 @@
 // The transfers of orctm_amd/csrc/nh_xfer.cpp on the host, over a runtime of this file's own in which device memory
-// is host memory and a copy is done when it is queued. Each check is an argument; prints OK.
+// is host memory, a copy is done when it is queued and a stream ends when the check says so. Each check is an argument; prints OK.
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
 
 #include <atomic>
+#include <chrono>
+#include <condition_variable>
 #include <future>
+#include <map>
+#include <mutex>
 #include <new>
 #include <set>
 #include <vector>
@@ -15,6 +19,12 @@
 static std::atomic<long> g_pins{0}, g_pin_limit{1 << 20}, g_copies{0};
 static std::atomic<bool> g_no_new{false};
 static thread_local hipError_t g_last = hipSuccess;
+static std::mutex g_mu;
+static std::condition_variable g_cv;
+static std::set<hipStream_t> g_busy;  // streams whose work has not ended
+static std::map<hipEvent_t, hipStream_t> g_at;
+static const hipStream_t kStuck = reinterpret_cast<hipStream_t>(8);
+static bool g_stuck = false;          // the copies on kStuck do not end
 static std::set<const void*> g_held;  // arrays pinned by the caller
 
 void* operator new(size_t n) {
@@ -53,9 +63,26 @@ hipError_t hipEventDestroy(hipEvent_t e) {
   free(e);
   return hipSuccess;
 }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t st) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  g_at[e] = st;
+  return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t st) {
+  std::unique_lock<std::mutex> lk(g_mu);
+  g_cv.wait(lk, [&] { return !g_busy.count(st); });
+  return hipSuccess;
+}
+hipError_t hipStreamQuery(hipStream_t st) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  return g_busy.count(st) ? g_last = hipErrorNotReady : hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t e) {
+  std::unique_lock<std::mutex> lk(g_mu);
+  const hipStream_t st = g_at[e];
+  g_cv.wait(lk, [&] { return !g_busy.count(st) && !(g_stuck && st == kStuck); });
+  return hipSuccess;
+}
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipGetLastError() {
   const hipError_t e = g_last;
@@ -195,11 +222,53 @@ static void held_by_the_runtime() {
   free(mem);
 }
 
+static bool ends(std::future<void>& f) { return f.wait_for(std::chrono::seconds(5)) == std::future_status::ready; }
+
+// A transfer whose stream is busy, and one whose copies are on their way, leave the others alone.
+static void side_by_side() {
+  const hipStream_t busy = reinterpret_cast<hipStream_t>(16);
+  const auto& s = kSizes[3];
+  xfer_retain();
+  g_busy.insert(busy);
+  auto waits = std::async(std::launch::async, [&] { round_trip(s.IE, s.JE, s.KE, s.flat, busy); });
+  std::this_thread::sleep_for(std::chrono::milliseconds(200));
+  auto other = std::async(std::launch::async, [&] { round_trip(s.IE, s.JE, s.KE, s.flat); });
+  const bool ended = ends(other);
+  {
+    std::lock_guard<std::mutex> lk(g_mu);
+    g_busy.clear();
+    g_cv.notify_all();
+  }
+  waits.wait();
+  other.wait();
+  need(ended, "a transfer beside one that waits for its stream");
+
+  const size_t n = 5000003;
+  const std::vector<double> a = numbers(n, 3.0), b = numbers(n, 5.0);
+  std::vector<double> x(n), y(n);
+  const XferPiece down = xfer_flat((void*)a.data(), x.data(), n * 8), up = xfer_flat(y.data(), b.data(), n * 8);
+  g_stuck = true;
+  auto first = std::async(std::launch::async, [&] { need(xfer_to_host(0, kStuck, &down, 1) == hipSuccess, "down"); });
+  std::this_thread::sleep_for(std::chrono::milliseconds(200));
+  auto second = std::async(std::launch::async, [&] { need(xfer_to_device(0, nullptr, &up, 1) == hipSuccess, "up"); });
+  const bool passed = ends(second);
+  {
+    std::lock_guard<std::mutex> lk(g_mu);
+    g_stuck = false;
+    g_cv.notify_all();
+  }
+  first.wait();
+  second.wait();
+  need(passed && x == a && y == b, "up beside down");
+  xfer_release();
+}
+
 int main(int argc, char** argv) {
   const char* what = argc > 1 ? argv[1] : "";
   if (!strcmp(what, "pin")) no_memory_to_pin();
   else if (!strcmp(what, "threads")) no_threads();
   else if (!strcmp(what, "held")) held_by_the_runtime();
+  else if (!strcmp(what, "beside")) side_by_side();
   else need(false, "an unknown check");
   printf("OK\n");
   return 0;
