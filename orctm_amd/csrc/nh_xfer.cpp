@@ -155,11 +155,14 @@ bool known(const void* host) {
 // The pieces through the runtime's own copies: flat ones queued, rows a plane at a time.
 hipError_t direct(hipStream_t st, const XferPiece* p, int n, bool to_host) {
   hipError_t e = hipSuccess;
+  bool flat = true;
   for (int q = 0; q < n && e == hipSuccess; ++q) {
+    flat = flat && p[q].flat();
     if (!p[q].flat()) continue;
     e = to_host ? hipMemcpyAsync(p[q].host, p[q].dev, p[q].bytes(), hipMemcpyDeviceToHost, st)
                 : hipMemcpyAsync(p[q].dev, p[q].host, p[q].bytes(), hipMemcpyHostToDevice, st);
   }
+  if (!to_host && e == hipSuccess && flat) return e;  // what is queued next follows; the caller waits for that anyway
   const hipError_t es = hipStreamSynchronize(st);
   if (e == hipSuccess) e = es;
   for (int q = 0; q < n; ++q) {

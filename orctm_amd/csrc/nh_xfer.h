@@ -52,7 +52,9 @@ XferPiece xfer_interior(void* dev, const void* host, int IE, int JE, int KE, siz
 
 // At most this many pieces in a call.
 constexpr int kXferPieces = 8;
-// Ordered on `st`; both return when every piece has arrived.
+// Ordered on `st`. To the host, it returns when every piece has arrived. To the device, work queued on `st` afterwards
+// finds the pieces there, and the caller waits for `st` before it gives the host arrays back (a wait of its own here
+// took 2 us of a small set_rhs's 36).
 hipError_t xfer_to_device(int device, hipStream_t st, const XferPiece* p, int n);
 hipError_t xfer_to_host(int device, hipStream_t st, const XferPiece* p, int n);
 

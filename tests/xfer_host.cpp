@@ -16,7 +16,7 @@
 
 #include "../orctm_amd/csrc/nh_xfer.cpp"
 
-static std::atomic<long> g_pins{0}, g_pin_limit{1 << 20}, g_copies{0};
+static std::atomic<long> g_pins{0}, g_pin_limit{1 << 20}, g_copies{0}, g_waits{0};
 static std::atomic<bool> g_no_new{false};
 static thread_local hipError_t g_last = hipSuccess;
 static std::mutex g_mu;
@@ -69,6 +69,7 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t st) {
   return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t st) {
+  ++g_waits;
   std::unique_lock<std::mutex> lk(g_mu);
   g_cv.wait(lk, [&] { return !g_busy.count(st); });
   return hipSuccess;
@@ -222,6 +223,16 @@ static void held_by_the_runtime() {
   free(mem);
 }
 
+// A small upload is queued and not waited for.
+static void queued() {
+  const std::vector<double> a = numbers(1000, 3.0);
+  std::vector<double> x(1000), y(1000);
+  const XferPiece two[2] = {xfer_flat(x.data(), a.data(), 8000), xfer_flat(y.data(), a.data(), 8000)};
+  xfer_retain();
+  need(xfer_to_device(0, nullptr, two, 2) == hipSuccess && g_copies == 2 && g_waits == 0 && x == a && y == a, "queued");
+  xfer_release();
+}
+
 static bool ends(std::future<void>& f) { return f.wait_for(std::chrono::seconds(5)) == std::future_status::ready; }
 
 // A transfer whose stream is busy, and one whose copies are on their way, leave the others alone.
@@ -269,6 +280,7 @@ int main(int argc, char** argv) {
   else if (!strcmp(what, "threads")) no_threads();
   else if (!strcmp(what, "held")) held_by_the_runtime();
   else if (!strcmp(what, "beside")) side_by_side();
+  else if (!strcmp(what, "queued")) queued();
   else need(false, "an unknown check");
   printf("OK\n");
   return 0;
