@@ -78,7 +78,12 @@ struct SorTb {
   static constexpr int PR = RY / 2;        // pair rows
   static constexpr int PL = RX * PR;       // cells per colour plane = pairs per region
   static constexpr int NP = PL / NT;       // pairs per thread
-  static constexpr int DP = 1;             // pair rows between consecutive pairs of a thread
+  // With a seam of an odd period and five pairs a thread, a cell loads all its factors and a block's wavefronts take
+  // pair rows in turn: the cells at the seam, loaded once more after the others, cost a launch more than the loads
+  // spared (T = 7, 1023 x 767 cells, periodic both ways: 1.35 ms a call, 1.44 with the neighbours' factors; 1023 x 768,
+  // along x: 1.31, 1.35). At two pairs a thread they do not (511 x 443, T = 12: 0.70 ms, 0.75 with all loads).
+  static constexpr bool OWN = SEAM && NP > 2;
+  static constexpr int DP = OWN ? NT / RX : 1;  // pair rows between consecutive pairs of a thread
   static constexpr int PAD = RX + 1;       // padding words before and after each plane
   static constexpr int PS = PL + 2 * PAD;  // plane stride
   static constexpr int BW = 2 * PS;        // start of the (B1O, SORPAR*FF) pairs, same plane order, no padding
@@ -114,7 +119,7 @@ struct SorTb {
   }
 
   __host__ __device__ static int at_least_2(int v) { return v < 2 ? 2 : v; }
-  __host__ __device__ static int pair_row(int tid, int k) { return tid / RX * NP + k; }
+  __host__ __device__ static int pair_row(int tid, int k) { return tid / RX * (OWN ? 1 : NP) + DP * k; }
 
   // Region origin (virtual coordinates of region cell (0, 0)) of tile t.
   __host__ __device__ static void origin(const TbGeom& g, int t, int& vx0, int& vy0) {
@@ -132,7 +137,8 @@ struct SorTb {
     r.m1 = 0u;
     r.s0 = (vx0 + x + vy0) & 1;
     TbCo co[NP][2];
-    double above = vf[v2(g, mi ? mi : 2, at_least_2(tb_map(vy0 + 2 * pair_row(tid, 0), g.JE, g.cyc_y)) - 1)];
+    double above = 0.0;
+    if constexpr (!OWN) above = vf[v2(g, mi ? mi : 2, at_least_2(tb_map(vy0 + 2 * pair_row(tid, 0), g.JE, g.cyc_y)) - 1)];
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
       const int p = pair_row(tid, k);
@@ -148,13 +154,15 @@ struct SorTb {
         const int zi = in ? mi : 2, zj = in ? mj : 2, ci = upd ? mi : 2, cj = upd ? mj : 2;
         const double zv = zin[p2(g, zi, zj)];
         const double b = b1o[p2(g, ci, cj)], f = ff[p2(g, ci, cj)];
-        const double ue = uf[u2(g, zi, zj)], vn = vf[v2(g, zi, zj)];
+        const int fi = OWN ? ci : zi, fj = OWN ? cj : zj;
+        const double ue = uf[u2(g, fi, fj)], vn = vf[v2(g, fi, fj)];
 #if defined(__HIP_DEVICE_COMPILE__)
         // lane 0 holds the region's first column, which is not updated
-        const double uw = RX == 64 ? __shfl_up(ue, 1, 64) : uf[u2(g, ci - 1, cj)];
+        const double uw = RX == 64 && !OWN ? __shfl_up(ue, 1, 64) : uf[u2(g, ci - 1, cj)];
 #else
         const double uw = uf[u2(g, ci - 1, cj)];
 #endif
+        if constexpr (OWN) above = vf[v2(g, ci, cj - 1)];
         r.z[k][s] = in ? zv : 0.0;
         lz[at(x, y)] = r.z[k][s];
         // SORPAR*FF(I,J) is the first product of the source's expression
@@ -167,7 +175,7 @@ struct SorTb {
         else r.m1 |= bit;
       }
     }
-    if (g.cyc_x || g.cyc_y) {  // across a seam the lane before and the row above are columns IE-1, JE-1, not 1
+    if (!OWN && (g.cyc_x || g.cyc_y)) {  // across a seam the lane before and the row above are columns IE-1, JE-1, not 1
 #pragma unroll
       for (int k = 0; k < NP; ++k)
 #pragma unroll
