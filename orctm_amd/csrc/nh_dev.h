@@ -203,16 +203,23 @@ __device__ __forceinline__ bool map_ij(int& i, int& j, int nx, int ny, int cx, i
 // of the assembly, bit for bit; float: the inner operator). c7: centre, W, E, N, S, U, D.
 // flags: bit 0 wet; bits 1-6 coupling present W E N S U D; bits 7-8 X_C variant (full, XUe*XP,
 // XUw*XP, 0); bits 9-10 Y_C variant (full, YVs*YP, YVn*YP, 0); bit 11 Z_C variant (full, ZW*ZP).
-template <typename T>
+// FLAT: one select after the other; a chain of ?: becomes branches, which empty the load pipeline of kernels that keep
+// many loads in flight. The same value either way.
+template <typename T, bool FLAT = false>
 __device__ __forceinline__ void row_coef(const T* cc, T zwk, T zwk1, T zpk, unsigned f, T* c7) {
   const T xw = cc[0], xe = cc[1], yn = cc[2], ys = cc[3];
   const unsigned xc = (f >> 7) & 3u, yc = (f >> 9) & 3u;
-  // one select after the other: a chain of ?: becomes branches, which empty the load pipeline
-  T X_C = xc == 2 ? xw : T(0), Y_C = yc == 2 ? yn : T(0);
-  X_C = xc == 1 ? xe : X_C;
-  X_C = xc == 0 ? cc[4] : X_C;
-  Y_C = yc == 1 ? ys : Y_C;
-  Y_C = yc == 0 ? cc[5] : Y_C;
+  T X_C, Y_C;
+  if constexpr (FLAT) {
+    X_C = xc == 2 ? xw : T(0), Y_C = yc == 2 ? yn : T(0);
+    X_C = xc == 1 ? xe : X_C;
+    X_C = xc == 0 ? cc[4] : X_C;
+    Y_C = yc == 1 ? ys : Y_C;
+    Y_C = yc == 0 ? cc[5] : Y_C;
+  } else {
+    X_C = xc == 0 ? cc[4] : xc == 1 ? xe : xc == 2 ? xw : T(0);
+    Y_C = yc == 0 ? cc[5] : yc == 1 ? ys : yc == 2 ? yn : T(0);
+  }
   const T Z_C = ((f >> 11) & 1u) ? zwk * zpk : (zwk + zwk1) * zpk;
   c7[0] = -(X_C + Y_C + Z_C);
   c7[1] = (f & (1u << 1)) ? xw : T(0);
@@ -287,24 +294,30 @@ struct ZCol {
     return d == 0 ? p0 : d == 1 ? p1 : d == 2 ? p2 : tp[m];
   }
   // the window's value at level m where the window covers m, else t (the table's entry)
+  template <bool FLAT = false>
   __device__ T zw_or(int m, T t) const {
-    const int d = m - kx;
-    t = d == 2 ? w2 : t;
-    t = d == 1 ? w1 : t;
-    return d == 0 ? w0 : t;
+    return pick<FLAT>(m - kx, w0, w1, w2, t);
   }
+  template <bool FLAT = false>
   __device__ T zp_or(int m, T t) const {
-    const int d = m - kx;
-    t = d == 2 ? p2 : t;
-    t = d == 1 ? p1 : t;
-    return d == 0 ? p0 : t;
+    return pick<FLAT>(m - kx, p0, p1, p2, t);
+  }
+  template <bool FLAT>
+  __device__ static T pick(int d, T v0, T v1, T v2, T t) {
+    if constexpr (FLAT) {
+      t = d == 2 ? v2 : t;
+      t = d == 1 ? v1 : t;
+      return d == 0 ? v0 : t;
+    } else {
+      return d == 0 ? v0 : d == 1 ? v1 : d == 2 ? v2 : t;
+    }
   }
 };
 
 // Inner operator row C = S * (-A), S = DLXP*DLYP/ZP, in T arithmetic from the T copies.
-template <typename T>
+template <typename T, bool FLAT = false>
 __device__ __forceinline__ void inner_row(const T* cc, T zwk, T zwk1, T zpk, unsigned f, T* c7) {
-  row_coef<T>(cc, zwk, zwk1, zpk, f, c7);
+  row_coef<T, FLAT>(cc, zwk, zwk1, zpk, f, c7);
   const T S = cc[6] / zpk;
 #pragma unroll
   for (int q = 0; q < 7; ++q) c7[q] = S * (-c7[q]);

@@ -588,7 +588,7 @@ __global__ __launch_bounds__(64 * H) void k_residual(const Sys* __restrict__ sys
       auto compute = [&](int k, const Lv& v) {
         const double xd = k < nz - 1 ? v.pd : 0.0;
         double c7[7];
-        row_coef<double>(cc, zwk, v.zw1, v.zp, v.f, c7);
+        row_coef<double, true>(cc, zwk, v.zw1, v.zp, v.f, c7);
         double a = c7[0] * x0;
         a = fma(c7[1], hw ? v.pw : 0.0, a);
         a = fma(c7[2], he ? v.pe : 0.0, a);
@@ -673,6 +673,12 @@ __global__ __launch_bounds__(64 * H) void k_refine(const Sys* __restrict__ syste
 //          Reads w l p_old x ZW ZP (+ 2 B of flags), writes p q x: 8 words + factor + 2 B per cell.
 // The halo lanes of k_bwd run the back-substitution recurrence of their halo columns themselves, so
 // z never goes to memory and no grid-wide step separates the two halves of the line solve.
+
+// Whether the matvec's rows are built with one select after the other (row_coef) or with branches. us per iteration
+// (matvec and column update), selects against branches: FP64 at 8 rows 512x443x49 262 and 245, 500x400x80 388 and 361,
+// 900x700x70 1104 and 1041 (mixed and 12 rows alike); at 4 rows 300x200x100 112 and 117, FP64 175 and 182.
+template <int H>
+constexpr bool kFlatRows = H == 4;
 
 // U: levels per load batch (the batch after next is loaded while one is computed).
 template <typename T, bool INIT, int H, int U>
@@ -1171,11 +1177,11 @@ void k_bwd(const Sys* __restrict__ systems, const Tile* __restrict__ tiles, int 
     T acc = T(0);
     if (centre) {
       const int b0 = k % 3;
-      const T zwk = (BUF && tab) ? zcol.zw_or(k, cur.tw) : cur.zw;
-      const T zpk = (BUF && tab) ? zcol.zp_or(k, cur.tp) : cur.zp;
+      const T zwk = (BUF && tab) ? zcol.template zw_or<true>(k, cur.tw) : cur.zw;
+      const T zpk = (BUF && tab) ? zcol.template zp_or<true>(k, cur.tp) : cur.zp;
       const unsigned fk = (BUF && derive) ? zcol.flag(k, nz) : cur.f;
       T c7[7];
-      inner_row<T>(cc, zwk, zw_below, zpk, fk, c7);
+      inner_row<T, kFlatRows<H>>(cc, zwk, zw_below, zpk, fk, c7);
       zw_below = zwk;
       acc = c7[0] * p0;
       acc = fmad(c7[1], lds[b0][sy][sx - 1], acc);
@@ -1363,7 +1369,7 @@ __global__ __launch_bounds__(bwd_threads<H>()) void k_bwd_ch(const Sys* __restri
           const T p0 = lds[b0][sy][sx];
           const T pm1 = k > 0 ? lds[(k - 1) & (NS - 1)][sy][sx] : T(0);
           T c7[7];
-          inner_row<T>(cc, rzw[u], zw_below, rzp[u], rf[u], c7);
+          inner_row<T, kFlatRows<H>>(cc, rzw[u], zw_below, rzp[u], rf[u], c7);
           zw_below = rzw[u];
           T acc = c7[0] * p0;
           acc = fmad(c7[1], lds[b0][sy][sx - 1], acc);

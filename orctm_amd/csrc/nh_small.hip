@@ -472,10 +472,10 @@ __global__ __launch_bounds__(NS) void k_mv(const Sys one, const Sys* __restrict_
       const int k = lev + LV * (u0 + u);
       if (u0 + u < U && k < nz) {
         const T* pc = Pl + k * LP + c + 1;
-        const T zwk = tab ? zcol.zw_or(k, rd[u].zw) : rd[u].zw, zwk1 = tab ? zcol.zw_or(k + 1, rd[u].zw1) : rd[u].zw1;
-        const T zpk = tab ? zcol.zp_or(k, rd[u].zp) : rd[u].zp;
+        const T zwk = tab ? zcol.template zw_or<true>(k, rd[u].zw) : rd[u].zw, zwk1 = tab ? zcol.template zw_or<true>(k + 1, rd[u].zw1) : rd[u].zw1;
+        const T zpk = tab ? zcol.template zp_or<true>(k, rd[u].zp) : rd[u].zp;
         T c7[7];
-        inner_row<T>(cc, zwk, zwk1, zpk, rd[u].f, c7);
+        inner_row<T, true>(cc, zwk, zwk1, zpk, rd[u].f, c7);
         T acc = c7[0] * pc[0];
         acc = fmad(c7[1], pc[-1], acc);
         acc = fmad(c7[2], pc[1], acc);

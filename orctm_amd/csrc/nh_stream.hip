@@ -449,11 +449,11 @@ __global__ __launch_bounds__(64 * H) void k_matvec(const Sys* __restrict__ syste
     for (int c = 0; c < V; ++c) {
       T pw = c == 0 ? west : pc[0], px = c == V - 1 ? east : pc[V - 1];
       if (WRAP) px = (c == 0 ? wrap_e0 : wrap_e1) ? po : px;
-      const T zwk = TAB ? zc[c].zw_or(k, r.tw) : tab ? zc[c].zw_or(k, r.tw) : get<T, V>(r.zw, c);
-      const T zpk = TAB ? zc[c].zp_or(k, r.tp) : tab ? zc[c].zp_or(k, r.tp) : get<T, V>(r.zp, c);
+      const T zwk = TAB ? zc[c].template zw_or<true>(k, r.tw) : tab ? zc[c].template zw_or<true>(k, r.tw) : get<T, V>(r.zw, c);
+      const T zpk = TAB ? zc[c].template zp_or<true>(k, r.tp) : tab ? zc[c].template zp_or<true>(k, r.tp) : get<T, V>(r.zp, c);
       T c7[7];
       if constexpr (TAB) inner_row<T>(cc[c], zwk, zwb[c], zpk, k, zc[c], c7);
-      else inner_row<T>(cc[c], zwk, zwb[c], zpk, V == 1 ? r.f : c ? r.f >> 16 : r.f & 0xffffu, c7);
+      else inner_row<T, true>(cc[c], zwk, zwb[c], zpk, V == 1 ? r.f : c ? r.f >> 16 : r.f & 0xffffu, c7);
       zwb[c] = zwk;
       T acc = c7[0] * pc[c];
       acc = fmad(c7[1], pw, acc);
