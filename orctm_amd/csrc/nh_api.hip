@@ -746,35 +746,58 @@ constexpr long long kSmallRows[2] = {512, 768};  // FP64, mixed
 // 192x160x35 (480) 52 against 43. Mixed at the same line as above: 192x192x45 (576) 44 against 49; 256x192x40 (768)
 // 44 against 44.
 constexpr long long kSmallRowsStream[2] = {256, 768};
+// Columns of few levels leave a block's wavefronts nothing to share out, and the line lies where every CU has its first
+// block (FP64) or its second (mixed). us per iteration, blocks against the streaming kernels, mixed: 512x50x4 (400
+// rows) 27 against 27, 512x65x2 (520) 33 against 29, 512x95x4 (760) 32 against 27, x16 28 against 26, x24 32 against
+// 31, x30 36 against 37. Against the tiled ones, FP64: 512x50x4 32 against 24, x8 32 against 27, 512x63x12 (504) 33
+// against 32, x16 34 against 37; mixed: 512x95x4 32 against 29, x12 29 against 30.
+constexpr int kFewLevelsStream = 16, kFewLevels[2] = {12, 8};  // FP64, mixed
+constexpr long long kSmallRowsFew[2] = {256, 512};
+// Without the table the streaming kernels have no depths to stop at and read the tiled ones' words. us per iteration,
+// tiled against streaming: mixed 201x203x13 28 against 30, 203x194x35 47 against 51, 191x259x64 75 against 86,
+// 300x250x60 88 against 97, 379x400x45 96 against 110, 700x600x30 163 against 172 (512x443x25, a width that the tiled
+// ones do not like, 92 against 83); FP64 203x194x35 (776 rows) 68 against 62, 191x259x64 117 against 101, 300x250x60
+// (1250) 151 against 157, 512x443x12 87 against 93, x49 263 against 296, 519x421x5 57 against 59. A context counts as
+// one without when most of its rows are: four of 256x256x50, one without, 8.1 ms a solve against 6.8, FP64 13.2
+// against 12.6.
+constexpr int kPlaneLevels[2] = {8, 16};              // FP64, mixed: up to as many levels they stream
+constexpr long long kPlaneRows[2] = {1200, 0};        // and up to as many rows
 // A single system of at most 64 rows takes blocks of 16 columns (up to 256 of them; 512x4x100 in blocks of 64:
-// 25 / 42 us); FP64 one of at most 128 rows and more than 56 levels blocks of 32 (1024x8x100: 43 against 61 us,
-// which has too many levels for the LDS of 64; 64x100x50: 32 against 31).
+// 25 / 42 us); FP64 one of at most 128 rows and more than 56 levels blocks of 32 (us, blocks of 64 against 32: 640x10
+// 31 against 34 at 56 levels, 45 against 35 at 64, 47 against 37 at 72; 80 and more do not fit the LDS of 64).
 constexpr long long kRows16 = 64, kRows32 = 128;
 constexpr int kLevels32 = 57;
 static_assert(kRows32 * 64 <= kSmallColumns, "the columns' sums are kept");
 
 // The kernels that the context's iterations run: blocks of columns (nh_small.h), the streaming ones (nh_stream.h), or
 // the tiled ones, which a forced tile height asks for, and which take what the streaming ones do not hold (more than
-// kStreamLevels levels, arrays past the reach of buffer descriptors).
-void ctx_form(Ctx& c, const std::vector<Sys>& systems, const std::vector<int>& forced) {
+// kStreamLevels levels, arrays past the reach of buffer descriptors) or are no better at (kPlaneLevels).
+void ctx_form(Ctx& c, const std::vector<Sys>& systems, const std::vector<int>& forced,
+              const std::vector<int>& zw_table) {
   SmallLaunch& l = c.rows;
-  long long rows = 0;
+  long long rows = 0, plane_rows = 0;
   c.nz = 0;
-  for (const Sys& s : systems) {
-    rows += (long long)s.tiles_x * s.ny;
+  for (int q = 0; q < c.nsys; ++q) {
+    const Sys& s = systems[q];
+    const long long n = (long long)s.tiles_x * s.ny;
+    rows += n;
+    if (!s.tab || zw_table[q] < 0) plane_rows += n;
     c.nz = std::max(c.nz, s.nz);
     c.any_wrap = c.any_wrap || s.cyc_x;
   }
   for (int h : forced)
     if (h > 0) return;
-  const bool stream = c.buf && c.nz <= kStreamLevels;
+  const int prec = c.fp32 ? 1 : 0;
+  const bool tiled = 2 * plane_rows > rows && c.nz > kPlaneLevels[prec] && rows > kPlaneRows[prec];
+  const bool stream = c.buf && c.nz <= kStreamLevels && !tiled;
+  const bool few = c.nz <= (stream ? kFewLevelsStream : kFewLevels[prec]);
   l.nz = c.nz;
   l.fp32 = c.fp32;
   l.nsys = c.nsys;
   l.one = c.nsys == 1;
   l.wc = !l.one || rows > kRows32 ? 64 : rows <= kRows16 ? 16 : !c.fp32 && l.nz >= kLevels32 ? 32 : 64;
   l.nblocks = (int)std::min(rows, kSmallRows[1]) * (64 / l.wc);
-  c.small = rows <= (stream ? kSmallRowsStream : kSmallRows)[c.fp32 ? 1 : 0] && small_fits(l.nz, c.fp32, l.wc);
+  c.small = rows <= (few ? kSmallRowsFew : stream ? kSmallRowsStream : kSmallRows)[prec] && small_fits(l.nz, c.fp32, l.wc);
   c.stream_form = stream && !c.small;
 }
 
@@ -812,7 +835,7 @@ hipError_t ctx_build(Ctx& c, const std::vector<Sys>& systems, const std::vector<
   for (const Sys& s : systems) c.cells += (long long)s.nx * s.ny * s.nz;
   c.fp32 = fp32;
   c.check_every = check_every > 0 ? check_every : 16;
-  ctx_form(c, systems, forced);
+  ctx_form(c, systems, forced, zw_table);
   c.max_outer = max_outer;
   c.device = device;
   for (const Sys& s : systems) c.maxit = std::max(c.maxit, s.maxit);
