@@ -128,7 +128,8 @@ typedef struct orctm_nh_stats {
   int32_t status;       /* enum orctm_nh_status of this solve */
   int32_t outer_iters;  /* FP64 refinement steps taken */
   int32_t inner_iters;  /* total inner PCG iterations */
-  int32_t tile_rows;    /* tile height the inner-iteration kernels ran with for this system */
+  int32_t tile_rows;    /* tile height the inner-iteration kernels ran with for this system (on blocks of
+                           columns, which have none: the height the tiled kernels would take) */
   double rel_res;       /* final ||b - A p||_2 / ||b||_2 in FP64 with the reference operator */
   double bnorm;         /* ||b||_2 */
   double solve_ms;      /* device time of the solve (HIP events), excluding host<->device copies */
@@ -136,7 +137,8 @@ typedef struct orctm_nh_stats {
   int32_t zw_table;     /* 1: the iteration kernels read ZW/ZP from the wet column's per-level table and
                            each column's 3-level window around its bottom (checked bit for bit at create);
                            0: from the per-cell planes */
-  int32_t buffer_addressing; /* 1: the matvec kernel addressed memory through buffer descriptors */
+  int32_t buffer_addressing; /* 1: the matvec kernel addressed memory through buffer descriptors (on blocks
+                           of columns, which use pointers: the tiled kernels would) */
   double reserved[3];
 } orctm_nh_stats_t;
 

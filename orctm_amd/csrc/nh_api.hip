@@ -619,6 +619,8 @@ struct TuneSet {
 // and the fastest assignment is kept. Both choices are cached for the life of the process and in
 // the tuning file (tune_path), keyed by device, precision, size class (ceil(log2) of the column
 // count; of the total for stage 2) and ceil(log2) of the number of systems.
+// A context on blocks of columns launches no tiles and gets no groups; several systems on them are not timed either
+// (a cohort of a new count class lost 3 to 6 ms by it), a single one makes its class's choice for larger contexts.
 // Tiles of 64 x 12 needed before a set of systems fills the device by itself (8 blocks per CU):
 // beyond it the tallest tile (fewest halo re-reads) is the fastest and no timing is run.
 constexpr long long kFillTiles = 8 * 256;
@@ -653,6 +655,7 @@ hipError_t ctx_heights(Ctx& c, const std::vector<Sys>& dev, const std::vector<in
       if (it != g_tune.end()) h = it->second;
     }
     if (!h && tiles12(dev, kv.second) >= kFillTiles) h = 12;
+    if (!h && c.small && c.nsys > 1) h = kTileHeights[0];
     if (!h) {
       TuneSet ts(c, dev, kv.second);
       HIPCHK(ts.upload());
@@ -671,6 +674,7 @@ hipError_t ctx_heights(Ctx& c, const std::vector<Sys>& dev, const std::vector<in
     }
     for (int q : kv.second) c.heights[q] = h;
   }
+  if (c.small) return hipSuccess;
   if (tuned.size() > 1 && classes.size() > 0) {
     // stage 2: the whole launch; code 0 = keep the per-class choice, else a uniform height
     const auto key = std::make_tuple(c.device, 100 + (c.fp32 ? 1 : 0), ceil_log2(cols), ceil_log2((long long)tuned.size()));
