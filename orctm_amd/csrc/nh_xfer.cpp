@@ -144,12 +144,12 @@ hipError_t work(Stage& s, int w, const Plan& plan, std::atomic<size_t>& next, bo
   return err;
 }
 
-// Whether the runtime holds the memory already: pinned or managed by the caller, or on a device.
-bool known(const void* host) {
+// What the runtime knows of the memory: pinned or managed by the caller, on a device, or nothing.
+hipMemoryType type_of(const void* host) {
   hipPointerAttribute_t a{};
-  if (hipPointerGetAttributes(&a, host) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+  if (hipPointerGetAttributes(&a, host) == hipSuccess) return a.type;
   (void)hipGetLastError();
-  return false;
+  return hipMemoryTypeUnregistered;
 }
 
 // The pieces through the runtime's own copies: flat ones queued, rows a plane at a time.
@@ -188,9 +188,13 @@ hipError_t transfer(int device, hipStream_t st, const XferPiece* p, int n, bool 
     flat = flat && p[q].flat();
   }
   if (flat && bytes < (to_host ? kXferDirectHost : kXferDirectDevice)) return direct(st, p, n, to_host);
-  bool held = flat || bytes >= kXferHeldRows;
-  for (int q = 0; q < n && held; ++q) held = known(p[q].host);
-  if (held) return direct(st, p, n, to_host);
+  bool held = flat || bytes >= kXferHeldRows, far = false;
+  for (int q = 0; q < n; ++q) {
+    const hipMemoryType t = type_of(p[q].host);
+    held = held && t != hipMemoryTypeUnregistered;
+    far = far || t == hipMemoryTypeDevice;  // not for the host's threads
+  }
+  if (held || far) return direct(st, p, n, to_host);
   const size_t part = (bytes / 12 + 7) / 8 * 8;
   const Plan plan(p, n, to_host ? std::min(std::max(part, kXferChunk / 8), kXferChunk) : kXferChunk);
   if (plan.chunks() == 0) return hipSuccess;

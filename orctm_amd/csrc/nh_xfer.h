@@ -15,6 +15,7 @@
 // the caller): the device reads and writes them itself (1024x768x60 to the device: 6.8 ms, 8.4 through the chunks;
 // 256x256x33: 0.35, 0.53), rows of an interior from kXferHeldRows on (to the host 7.1 ms, 7.5 through the chunks;
 // below, the copy commands of the levels cost more than the chunks: 400x300x40 0.98 ms, 0.88; 128x128x30 0.29, 0.17).
+// A piece whose host side lies on a device goes to the runtime's copies at any size: no thread of the host touches it.
 // The pinned buffers (kXferWorkers * 2 chunks, 32 MiB) and their events belong to the device, one set for each
 // direction in use, held by one transfer at a time and only while its copies run, not while it waits for kernels (two
 // threads of 1024x768 surfaces: 2.4 ms a solve each, 3.2 while it was held over the sweeps); they are freed with the process's last handle. Where no

@@ -4,6 +4,7 @@ runtime of the harness's own (tests/xfer_host.cpp): what arrives where, and what
 * only some of the chunks, or none, can be pinned (``pin``): fewer workers, or the runtime's own copies;
 * no thread can be started (``threads``): the caller does all the work;
 * the runtime holds the caller's arrays already (``held``): its copies take them as they are;
+* an array lies on the device (``device``): no thread of the host touches it;
 * others transfer too (``beside``): none waits for another's kernels, nor for another's copies the other way;
 * an upload is small (``queued``): it is left to the stream, which the caller waits for.
 """
@@ -27,7 +28,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["pin", "threads", "held", "beside", "queued"])
+@pytest.mark.parametrize("check", ["pin", "threads", "held", "device", "beside", "queued"])
 def test_transfer(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.strip() == "OK", r.stdout + r.stderr

@@ -26,6 +26,7 @@ static std::map<hipEvent_t, hipStream_t> g_at;
 static const hipStream_t kStuck = reinterpret_cast<hipStream_t>(8);
 static bool g_stuck = false;          // the copies on kStuck do not end
 static std::set<const void*> g_held;  // arrays pinned by the caller
+static const char* g_far = nullptr;   // an array on the device
 
 void* operator new(size_t n) {
   if (g_no_new) throw std::bad_alloc();
@@ -91,6 +92,10 @@ hipError_t hipGetLastError() {
   return e;
 }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
+  if (g_far && p >= g_far && p < g_far + (size_t(1) << 28)) {
+    a->type = hipMemoryTypeDevice;
+    return hipSuccess;
+  }
   for (const void* h : g_held)
     if (p >= h && p < (const char*)h + (size_t(1) << 30)) {
       a->type = hipMemoryTypeHost;
@@ -223,6 +228,32 @@ static void held_by_the_runtime() {
   free(mem);
 }
 
+// An array on the device in the place of the caller's is left to the runtime, whatever its size.
+static void on_the_device() {
+  xfer_retain();
+  char* mem = (char*)calloc(size_t(1) << 28, 1);
+  double* to = (double*)mem;
+  g_far = mem;
+  for (size_t KE : {1, 10, 100}) {
+    const size_t IE = 402, JE = 302, pitch = 416, plane = pitch * 300;
+    const std::vector<double> box = numbers(plane * KE, 0.5 + (double)KE);
+    const XferPiece p = xfer_interior((void*)box.data(), to, IE, JE, (int)KE, pitch, plane);
+    need(xfer_to_host(0, nullptr, &p, 1) == hipSuccess && g_pins == 0, "rows to the device's memory");
+    for (size_t k = 0; k < KE; ++k)
+      for (size_t j = 0; j < JE - 2; ++j)
+        need(!memcmp(to + 1 + IE * (j + 1 + JE * k), box.data() + plane * k + pitch * j, (IE - 2) * 8), "their values");
+  }
+  const size_t n = 3000003;
+  const std::vector<double> a = numbers(n, 3.0);
+  std::vector<double> x(n);
+  const XferPiece two[2] = {xfer_flat((void*)a.data(), to, n * 8), xfer_flat((void*)a.data(), x.data(), n * 8)};
+  need(xfer_to_host(0, nullptr, two, 2) == hipSuccess && g_pins == 0 && !memcmp(to, a.data(), n * 8) && x == a,
+       "one of two on the device");
+  xfer_release();
+  g_far = nullptr;
+  free(mem);
+}
+
 // A small upload is queued and not waited for.
 static void queued() {
   const std::vector<double> a = numbers(1000, 3.0);
@@ -279,6 +310,7 @@ int main(int argc, char** argv) {
   if (!strcmp(what, "pin")) no_memory_to_pin();
   else if (!strcmp(what, "threads")) no_threads();
   else if (!strcmp(what, "held")) held_by_the_runtime();
+  else if (!strcmp(what, "device")) on_the_device();
   else if (!strcmp(what, "beside")) side_by_side();
   else if (!strcmp(what, "queued")) queued();
   else need(false, "an unknown check");
