@@ -561,6 +561,9 @@ int orctm_nh_troneu(orctm_nh_sor_t* s, const double* u1o, const double* uzo, con
                           xfer_flat(s->a.b1o, b1o, p2 * 8)};
   // the source recomputes B1O on J = J_start+1..JE, I = I_start+1..IE: all of it where both start at 0
   hipError_t e = xfer_to_device(s->g.device, st, in, d.IS == 0 && d.JS == 0 ? 4 : 5);
+  // a few microseconds' kernels behind small copies that nobody waits for start late (a call of 512 x 4 cells 254 us,
+  // 231 so; 200 x 5: 189, 182); behind the blocked launches' graph the wait costs more (300 x 250: 691, 701)
+  if (e == hipSuccess && s->one) e = hipStreamSynchronize(st);
   if (e == hipSuccess) e = hipEventRecord(s->ev0, st);
   if (e == hipSuccess) {
     const long long nb = (long long)(d.IE - d.IS) * (d.JE - d.JS);
