@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <atomic>
 #include <mutex>
+#include <optional>
 #include <thread>
 
 #include "nh_lock.h"
@@ -14,15 +15,44 @@ namespace onh {
 namespace {
 
 struct Stage {
-  std::mutex mu;  // held for a transfer; taken after device_lock() where both are
+  bool taken = false;  // by a transfer, under Device::pick
   int device = -1;
   char* buf[kXferWorkers][2] = {};
   hipEvent_t ev[kXferWorkers][2] = {};
 };
 
-constexpr int kStages = 16;  // device ordinals beyond share them
-Stage g_stage[2][kStages];   // to the device, to the host
+// One transfer to the device and one to the host at a time, each with a stage of its own: the first while it is free,
+// so that a program that has one transfer under way at a time pins and gives back one stage.
+struct Device {
+  std::mutex way[2];  // to the device, to the host: held for a transfer; taken after device_lock() where both are
+  std::mutex pick;
+  Stage stage[2];
+};
+
+constexpr int kDevices = 16;  // device ordinals beyond share them
+Device g_device[kDevices];
 std::mutex g_count_mu;
+
+// A stage for the holder of a way, given back at the end of the scope.
+class Taken {
+ public:
+  explicit Taken(Device& d) : d_(d) {
+    std::lock_guard<std::mutex> lk(d.pick);
+    s_ = d.stage[0].taken ? &d.stage[1] : &d.stage[0];
+    s_->taken = true;
+  }
+  ~Taken() {
+    std::lock_guard<std::mutex> lk(d_.pick);
+    s_->taken = false;
+  }
+  Taken(const Taken&) = delete;
+  Taken& operator=(const Taken&) = delete;
+  Stage& stage() { return *s_; }
+
+ private:
+  Device& d_;
+  Stage* s_;
+};
 int g_handles = 0;
 
 // Workers whose buffers and events are there.
@@ -207,16 +237,22 @@ hipError_t transfer(int device, hipStream_t st, const XferPiece* p, int n, bool 
     es = hipStreamSynchronize(st);
   }
   if (es != hipSuccess) return es;
-  Stage& s = g_stage[to_host][(unsigned)device % kStages];
-  std::unique_lock<std::mutex> lk(s.mu);
-  if (made(s, device) < want) {  // allocates: not while another thread captures a graph
+  Device& d = g_device[(unsigned)device % kDevices];
+  std::unique_lock<std::mutex> lk(d.way[to_host]);
+  std::optional<Taken> at;  // given back before the way
+  at.emplace(d);
+  if (made(at->stage(), device) < want) {  // allocates: not while another thread captures a graph
+    at.reset();
     lk.unlock();
     std::lock_guard<std::recursive_mutex> dev(device_lock());
     lk.lock();
-    make(s, want, device);
+    at.emplace(d);
+    make(at->stage(), want, device);
   }
+  Stage& s = at->stage();
   want = std::min(want, made(s, device));
   if (want == 0) {  // no memory to pin
+    at.reset();
     lk.unlock();
     return direct(st, p, n, to_host);
   }
@@ -284,11 +320,11 @@ void xfer_release() {
   std::lock_guard<std::recursive_mutex> dev(device_lock());
   std::lock_guard<std::mutex> lk(g_count_mu);
   if (--g_handles > 0) return;
-  for (auto& way : g_stage)
-    for (Stage& s : way) {
-      std::lock_guard<std::mutex> ls(s.mu);
+  for (Device& d : g_device) {
+    std::scoped_lock ways(d.way[0], d.way[1]);
+    for (Stage& s : d.stage)
       if (s.device >= 0) drop(s);
-    }
+  }
 }
 
 }  // namespace onh

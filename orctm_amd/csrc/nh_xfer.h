@@ -16,10 +16,12 @@
 // 256x256x33: 0.35, 0.53), rows of an interior from kXferHeldRows on (to the host 7.1 ms, 7.5 through the chunks;
 // below, the copy commands of the levels cost more than the chunks: 400x300x40 0.98 ms, 0.88; 128x128x30 0.29, 0.17).
 // A piece whose host side lies on a device goes to the runtime's copies at any size: no thread of the host touches it.
-// The pinned buffers (kXferWorkers * 2 chunks, 32 MiB) and their events belong to the device, one set for each
-// direction in use, held by one transfer at a time and only while its copies run, not while it waits for kernels (two
-// threads of 1024x768 surfaces: 2.4 ms a solve each, 3.2 while it was held over the sweeps); they are freed with the process's last handle. Where no
-// memory can be pinned, a transfer works with as many workers as have their buffers, or through the runtime.
+// The pinned buffers (kXferWorkers * 2 chunks, 32 MiB) and their events belong to the device. One transfer each way is
+// under way at a time, and only while its copies run, not while it waits for kernels (two threads of 1024x768 surfaces:
+// 2.4 ms a solve each, 3.2 while it was held over the sweeps); a second set of buffers is made where both ways meet (a
+// set for each way cost a program that closes its last handle 6 ms of the next one's making, 323x293x42). They are
+// freed with the process's last handle. Where no memory can be pinned, a transfer works with as many workers as have
+// their buffers, or through the runtime.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -6,6 +6,7 @@ runtime of the harness's own (tests/xfer_host.cpp): what arrives where, and what
 * the runtime holds the caller's arrays already (``held``): its copies take them as they are;
 * an array lies on the device (``device``): no thread of the host touches it;
 * others transfer too (``beside``): none waits for another's kernels, nor for another's copies the other way;
+* transfers go one after the other (``stage``): they share one set of chunks, both ways;
 * an upload is small (``queued``): it is left to the stream, which the caller waits for.
 """
 import os
@@ -28,7 +29,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["pin", "threads", "held", "device", "beside", "queued"])
+@pytest.mark.parametrize("check", ["pin", "threads", "held", "device", "beside", "stage", "queued"])
 def test_transfer(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.strip() == "OK", r.stdout + r.stderr

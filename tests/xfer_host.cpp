@@ -305,6 +305,15 @@ static void side_by_side() {
   xfer_release();
 }
 
+// A program with one transfer under way at a time pins one stage, both ways.
+static void one_stage() {
+  xfer_retain();
+  for (int q = 0; q < 2; ++q) round_trip(kSizes[4].IE, kSizes[4].JE, kSizes[4].KE, kSizes[4].flat);
+  need(g_pins == 2 * kXferWorkers, "one stage");
+  xfer_release();
+  need(g_pins == 0, "given back");
+}
+
 int main(int argc, char** argv) {
   const char* what = argc > 1 ? argv[1] : "";
   if (!strcmp(what, "pin")) no_memory_to_pin();
@@ -312,6 +321,7 @@ int main(int argc, char** argv) {
   else if (!strcmp(what, "held")) held_by_the_runtime();
   else if (!strcmp(what, "device")) on_the_device();
   else if (!strcmp(what, "beside")) side_by_side();
+  else if (!strcmp(what, "stage")) one_stage();
   else if (!strcmp(what, "queued")) queued();
   else need(false, "an unknown check");
   printf("OK\n");
