@@ -140,39 +140,58 @@ hipError_t device_half(const Chunk& c, char* buf, bool to_host, hipStream_t st) 
 }
 
 // One worker: chunks from the common counter through its two buffers. Every copy that it issued has
-// finished when it returns.
-hipError_t work(Stage& s, int w, const Plan& plan, std::atomic<size_t>& next, bool to_host, hipStream_t st) {
-  hipError_t err = hipSuccess;
-  Chunk held[2];
-  bool pending[2] = {false, false};
-  auto settle = [&](int q) {
-    if (!pending[q]) return;
-    pending[q] = false;
-    const hipError_t e = hipEventSynchronize(s.ev[w][q]);
-    if (err == hipSuccess) err = e;
-    if (to_host && e == hipSuccess) host_copy(held[q], s.buf[w][q], true);
-  };
-  const size_t n = plan.chunks();
-  int q = 0;
-  for (size_t k = next++; k < n && err == hipSuccess; k = next++) {
+// finished when run() returns.
+class Worker {
+ public:
+  Worker(Stage& s, int w, const Plan& plan, std::atomic<size_t>& next, bool to_host, hipStream_t st)
+      : s_(s), w_(w), plan_(plan), next_(next), to_host_(to_host), st_(st) {}
+  // The next chunk's copies, into a buffer that is not in use any more; false: no chunk left, or an error.
+  bool issue() {
+    if (err_ != hipSuccess) return false;
+    const size_t k = next_++;
+    if (k >= plan_.chunks()) return false;
+    const int q = q_;
     settle(q);
-    held[q] = plan.chunk(k);
-    if (!to_host) host_copy(held[q], s.buf[w][q], false);
-    hipError_t e = device_half(held[q], s.buf[w][q], to_host, st);
-    if (e == hipSuccess) e = hipEventRecord(s.ev[w][q], st);
+    held_[q] = plan_.chunk(k);
+    if (!to_host_) host_copy(held_[q], s_.buf[w_][q], false);
+    hipError_t e = device_half(held_[q], s_.buf[w_][q], to_host_, st_);
+    if (e == hipSuccess) e = hipEventRecord(s_.ev[w_][q], st_);
     if (e == hipSuccess) {
-      pending[q] = true;
+      pending_[q] = true;
     } else {
-      hipStreamSynchronize(st);  // a copy without an event may still use the buffer
-      err = e;
+      hipStreamSynchronize(st_);  // a copy without an event may still use the buffer
+      err_ = e;
     }
-    q ^= 1;
-    if (to_host) settle(q);  // the chunk before, while this one is on its way
+    q_ ^= 1;
+    return true;
   }
-  settle(q);
-  settle(q ^ 1);
-  return err;
-}
+  hipError_t run() {
+    while (issue())
+      if (to_host_) settle(q_);  // the chunk before, while this one is on its way
+    settle(q_);
+    settle(q_ ^ 1);
+    return err_;
+  }
+
+ private:
+  void settle(int q) {
+    if (!pending_[q]) return;
+    pending_[q] = false;
+    const hipError_t e = hipEventSynchronize(s_.ev[w_][q]);
+    if (err_ == hipSuccess) err_ = e;
+    if (to_host_ && e == hipSuccess) host_copy(held_[q], s_.buf[w_][q], true);
+  }
+  Stage& s_;
+  const int w_;
+  const Plan& plan_;
+  std::atomic<size_t>& next_;
+  const bool to_host_;
+  const hipStream_t st_;
+  hipError_t err_ = hipSuccess;
+  Chunk held_[2];
+  bool pending_[2] = {false, false};
+  int q_ = 0;
+};
 
 // What the runtime knows of the memory: pinned or managed by the caller, on a device, or nothing.
 hipMemoryType type_of(const void* host) {
@@ -259,17 +278,19 @@ hipError_t transfer(int device, hipStream_t st, const XferPiece* p, int n, bool 
   std::atomic<size_t> next{0};
   hipError_t got[kXferWorkers] = {};
   std::thread team[kXferWorkers];
+  Worker self(s, 0, plan, next, to_host, st);
+  if (to_host && self.issue()) self.issue();  // on their way while the others are made
   for (int w = 1; w < want; ++w) {
     try {
       team[w] = std::thread([&, w] {
         const hipError_t e = hipSetDevice(device);
-        got[w] = e == hipSuccess ? work(s, w, plan, next, to_host, st) : e;
+        got[w] = e == hipSuccess ? Worker(s, w, plan, next, to_host, st).run() : e;
       });
     } catch (...) {
       break;  // no thread or no memory for one to be had: the others take its share
     }
   }
-  got[0] = work(s, 0, plan, next, to_host, st);
+  got[0] = self.run();
   for (std::thread& t : team)
     if (t.joinable()) t.join();
   for (hipError_t e : got)
