@@ -234,12 +234,17 @@ int alloc_state(orctm_nh_t* h) {
   SALLOC(pa, NP * es, void*);
   SALLOC(pb, NP * es, void*);
   SALLOC(q, NP * es, void*);
-  SALLOC(use, (size_t)h->plane * sizeof(int), int*);
-  SALLOC(partials, 2 * (size_t)s.nslots * sizeof(double), double*);
-  // sums of nh_small.hip: per 64-column row, or per column where a block may take fewer
+  // the small arrays in one allocation: each of its own took 12 us of a clone
   const size_t rows64 = (size_t)s.tiles_x * s.ny;
-  SALLOC(rowsum, 4 * rows64 * (rows64 * 64 <= (size_t)kSmallColumns ? 64 : 1) * es, void*);
-  SALLOC(nbp, sizeof(double), double*);
+  // sums of nh_small.hip: per 64-column row, or per column where a block may take fewer
+  const size_t sums = 4 * rows64 * (rows64 * 64 <= (size_t)kSmallColumns ? 64 : 1) * es;
+  const size_t sizes[] = {2 * (size_t)s.nslots * sizeof(double), sums, sizeof(double), (size_t)h->plane * sizeof(int)};
+  size_t at[5] = {0};
+  for (int q = 0; q < 4; ++q) at[q + 1] = at[q] + (sizes[q] + 255) / 256 * 256;
+  SALLOC(partials, at[4], double*);
+  s.rowsum = reinterpret_cast<char*>(s.partials) + at[1];
+  s.nbp = reinterpret_cast<double*>(reinterpret_cast<char*>(s.partials) + at[2]);
+  s.use = reinterpret_cast<int*>(reinterpret_cast<char*>(s.partials) + at[3]);
 #undef SALLOC
   h->d_nb = s.nbp;
   return ORCTM_NH_OK;
@@ -1648,7 +1653,8 @@ int orctm_nh_inner_apply(orctm_nh_t* h, const void* x, void* y) {
   }
   const size_t es = h->fp32 ? 4 : 8;
   Ctx& c = h->ctx;
-  // x goes where the forward elimination leaves w; the matvec kernel in raw mode takes it as z
+  // x goes to z, which the blocks of columns' and the streaming matvec read; the tiled one, in raw mode, takes it in the
+  // place of the forward elimination's w
   hipError_t e = hipMemset(h->sys.z, 0, (size_t)h->plane * h->nz * es);
   if (e == hipSuccess) e = hipDeviceSynchronize();
   if (e == hipSuccess) e = to_device_vec(h, h->sys.z, x, es);
@@ -1685,8 +1691,8 @@ int orctm_nh_inner_precond(orctm_nh_t* h, const void* r, void* z, double* rho) {
   }
   const size_t es = h->fp32 ? 4 : 8;
   Ctx& c = h->ctx;
-  // forward elimination (init kernel) then back substitution inside the matvec kernel, whose first
-  // iteration writes p = z into search-direction buffer B
+  // the first column update and the first matvec: the line solve is in the former (blocks of columns, streaming) or
+  // shared by both (tiled); the matvec's first iteration writes p = z into search-direction buffer B
   Outer o{};
   o.odone = RUN;
   hipError_t e = hipMemcpy(c.d_outer, &o, sizeof(o), hipMemcpyHostToDevice);
