@@ -391,6 +391,8 @@ def bench_batch(args):
         g, divg = synth.build(sp)
         systems.append((g, divg))
     cells = sum(g.cells for g, _ in systems)
+    streaming = args.tile_rows == 0 and args.buffer_addressing == 0 and args.zw_table == 0
+    work = [cells_in_use(g, 4) if streaming else g.cells for g, _ in systems]
     log(f"[bench] batch: {len(systems)} systems, {cells} cells, generated in {time.perf_counter() - t:.1f} s")
     out = {}
     precs = (("mixed", abi.MIXED), ("fp64", abi.FP64))
@@ -431,7 +433,7 @@ def bench_batch(args):
         inner = sum(x["inner_iters"] for x in st)
         # cell-iterations actually processed per solve (converged systems drop out of later launches)
         cell_iters = sum(x["inner_iters"] * g.cells for x, (g, _) in zip(st, systems))
-        mv_bytes = sum(x["inner_iters"] * MATVEC_BYTES[4] * g.cells for x, (g, _) in zip(st, systems))
+        mv_bytes = sum(x["inner_iters"] * MATVEC_BYTES[4] * w for x, w in zip(st, work))
         # one-by-one reference timing of the same systems (sequential, same kernels)
         t1 = time.perf_counter()
         for s in solvers:
@@ -481,9 +483,9 @@ def bench_batch(args):
         "device": device_state(),
         "roofline": {"bound": "hbm", "kernel": "inner matvec, FP32 (batched)", "achieved": round(mv_gbs, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(mv_gbs / HBM_PEAK_GBS, 4),
-                     "traffic": traffic, "bytes_per_launch": MATVEC_BYTES[4] * cells,
-                     "note": "the bare matvec bytes (36 B per cell of the box, dry ones that the kernels skip too, FP32) per "
-                             "active cell-iteration over the "
+                     "traffic": traffic, "bytes_per_launch": MATVEC_BYTES[4] * sum(work), "cells_in_use": sum(work),
+                     "note": "the bare matvec bytes (36 B per cell of the levels in use, FP32) per active "
+                             "cell-iteration over the "
                              "summed matvec launch time; bytes_per_launch and traffic (HBM bytes counted by "
                              "FETCH_SIZE/WRITE_SIZE) are those of one launch in which every system iterates"},
         "cpu_baseline": None,

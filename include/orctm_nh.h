@@ -98,7 +98,8 @@ typedef struct orctm_nh_options {
                            than 16 levels, FP64 more than 8 in more than 1200 rows of 64 columns) on tiled
                            kernels tuned per size class at create / batch create.
                            4, 8 or 12 = the tiled kernels at that height. Results are the same bits
-                           for every choice (block sums are formed over fixed 4-row groups). Tuned picks
+                           for every choice (block sums are formed over fixed 4-row groups; the sign of a
+                           zero that a first guess has on land apart). Tuned picks
                            persist per device (arch/CU count), precision and size class in a JSON file:
                            $ORCTM_NH_TUNE_FILE (set but empty: none), else
                            $XDG_CACHE_HOME/orctm_nh/tile_tuning.json, else

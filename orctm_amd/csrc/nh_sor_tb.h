@@ -17,13 +17,13 @@
 // result; across a cyclic seam with an odd period a neighbour can share the colour, and the source then
 // reads the halo copy, which also holds the value from before the half-sweep.
 //
-// Work split. A thread owns NP vertical pairs (x, 2p) and (x, 2p+1), one below the other, one cell of each
-// colour, so every lane updates one cell per half-sweep; consecutive lanes own consecutive x, so the region
-// loads and the tile stores are contiguous rows. VF(J-1) of a cell is VF(J) of the cell above it, which the
-// thread has loaded for all but its first pair, and UF(I-1) is UF(I) of the lane before (on the device, RX =
-// 64): 10.2 loads a pair instead of 14 (NP = 5), of the 72 MB that a launch over 1026 x 770 cells brought in. The LDS holds the region split by colour: plane (x + y) & 1,
-// row y >> 1, column x, padded by a row and a word on either side, so the four neighbours of a cell lie
-// in the other plane, consecutive lanes read consecutive words, and a lane's reads for all its pairs
+// Work split. A thread owns NP vertical pairs (x, 2p) and (x, 2p+1), one below the other, one cell of each colour, so
+// every lane updates one cell per half-sweep; consecutive lanes own consecutive x, so the region loads and the tile
+// stores are contiguous rows. VF(J-1) of a cell is VF(J) of the cell above it, which the thread has loaded for all
+// but its first pair, and UF(I-1) is UF(I) of the lane before (on the device, RX = 64): 10.2 loads a pair instead of
+// 14 (NP = 5), of the 72 MB that a launch over 1026 x 770 cells brought in. The LDS holds the region split by colour:
+// plane (x + y) & 1, row y >> 1, column x, padded by a row and a word on either side, so the four neighbours of a
+// cell lie in the other plane, consecutive lanes read consecutive words, and a lane's reads for all its pairs
 // are one base address plus constant offsets. B1O and SORPAR*FF of every cell sit beside them in LDS;
 // the four face coefficients of a thread's cells stay in registers for the whole launch, ordered by
 // the colour that updates them, which keeps a 512-thread block within 256 VGPRs at five pairs per thread.

@@ -8,9 +8,10 @@
 // What bounds them is memory: 1024x768x60 in FP32 runs at 4.9 TB/s of a copy's 6.1 with every level read. So each
 // column stops at the levels in use (Sys::use): its depth, or what r holds below it, made equal over 64 bytes of a
 // row so that stores fill whole pieces. Dry cells have no couplings: where r is 0 the rest of their vectors is 0 and
-// adds nothing to a sum, hence the same bits. The other loss was the pipeline of loads, which a chain of ?: or an exit
-// in the middle of the loop empties (the compiler waits for every load where paths meet): selects one after the
-// other, whole turns of the ring of levels, and the loads of a level fixed in place before its arithmetic.
+// adds nothing to a sum, hence the same values (a zero's sign apart). The other loss was the pipeline of loads, which
+// a chain of ?: or an exit in the middle of the loop empties (the compiler waits for every load where paths meet):
+// selects one after the other, whole turns of the ring of levels, and the loads of a level fixed in place before its
+// arithmetic.
 //
 // us per iteration (matvec + update), tiled -> these, on basins of 0.5 to 0.6 wet cells: 1024x768x60 mixed 270 + 168
 // -> 220 + 156, FP64 535 + 429 -> 429 + 336; 512x443x49 74 + 65 -> 62 + 41, FP64 144 + 90 -> 116 + 87; 203x194x35
