@@ -771,6 +771,15 @@ constexpr long long kSmallRowsFew[2] = {256, 512};
 // against 12.6.
 constexpr int kPlaneLevels[2] = {8, 16};              // FP64, mixed: up to as many levels they stream
 constexpr long long kPlaneRows[2] = {1200, 0};        // and up to as many rows
+// Columns of one or two levels are outweighed by what the streaming matvec loads once a column, and FP64 columns of few
+// levels in a channel of at most two tiles by the rows that blocks of 4 read twice. us per iteration, tiled against
+// streaming, from the rows at which they lose (below, they are as quick or quicker): one level, 300x420 (2100 rows) 43
+// and 43, FP64 38 and 40, 1000x1000 84 and 97, 104 and 136; two, 500x800 (6400) 50 and 53, 66 and 69, 1000x2400 164
+// and 180, 274 and 315 (three alike, four 202 and 205, 368 and 360); FP64 channels, 10x6000x4 46 and 54, x9 64 and
+// 71, x12 73 and 75, 90x3000x4 61 and 65, 64x6000x9 96 and 95.
+bool shallow(int nz, bool fp32, long long rows, long long narrow_rows) {
+  return nz == 1 ? rows > 2000 : nz == 2 ? rows > 3100 : !fp32 && nz <= 9 && rows > 5000 && 2 * narrow_rows > rows;
+}
 // A single system of at most 64 rows takes blocks of 16 columns (up to 256 of them; 512x4x100 in blocks of 64:
 // 25 / 42 us); FP64 one of at most 128 rows and more than 56 levels blocks of 32 (us, blocks of 64 against 32: 640x10
 // 31 against 34 at 56 levels, 45 against 35 at 64, 47 against 37 at 72; 80 and more do not fit the LDS of 64).
@@ -780,24 +789,26 @@ static_assert(kRows32 * 64 <= kSmallColumns, "the columns' sums are kept");
 
 // The kernels that the context's iterations run: blocks of columns (nh_small.h), the streaming ones (nh_stream.h), or
 // the tiled ones, which a forced tile height asks for, and which take what the streaming ones do not hold (more than
-// kStreamLevels levels, arrays past the reach of buffer descriptors) or are no better at (kPlaneLevels).
+// kStreamLevels levels, arrays past the reach of buffer descriptors) or are no better at (kPlaneLevels, shallow).
 void ctx_form(Ctx& c, const std::vector<Sys>& systems, const std::vector<int>& forced,
               const std::vector<int>& zw_table) {
   SmallLaunch& l = c.rows;
-  long long rows = 0, plane_rows = 0;
+  long long rows = 0, plane_rows = 0, narrow_rows = 0;
   c.nz = 0;
   for (int q = 0; q < c.nsys; ++q) {
     const Sys& s = systems[q];
     const long long n = (long long)s.tiles_x * s.ny;
     rows += n;
     if (!s.tab || zw_table[q] < 0) plane_rows += n;
+    if (s.tiles_x <= 2) narrow_rows += n;
     c.nz = std::max(c.nz, s.nz);
     c.any_wrap = c.any_wrap || s.cyc_x;
   }
   for (int h : forced)
     if (h > 0) return;
   const int prec = c.fp32 ? 1 : 0;
-  const bool tiled = 2 * plane_rows > rows && c.nz > kPlaneLevels[prec] && rows > kPlaneRows[prec];
+  const bool tiled = (2 * plane_rows > rows && c.nz > kPlaneLevels[prec] && rows > kPlaneRows[prec]) ||
+                     shallow(c.nz, c.fp32, rows, narrow_rows);
   const bool stream = c.buf && c.nz <= kStreamLevels && !tiled;
   const bool few = c.nz <= (stream ? kFewLevelsStream : kFewLevels[prec]);
   l.nz = c.nz;
