@@ -95,8 +95,8 @@ typedef struct orctm_nh_options {
   int32_t tile_rows;    /* rows (j) per tile of the inner-iteration kernels: 0 (default) = chosen by size:
                            launches of few columns run on blocks of columns and those of many, up to 64
                            levels, on streaming kernels of 4 rows; the rest (without the ZW/ZP table: more
-                           than 16 levels, FP64 more than 8 in more than 1200 rows of 64 columns; one or
-                           two levels in thousands of rows) on tiled kernels tuned per size class at
+                           than 16 levels, FP64 more than 8 in more than 1200 rows of 64 columns or any in
+                           more than 4000; one or two levels in thousands of rows) on tiled kernels tuned per size class at
                            create / batch create.
                            4, 8 or 12 = the tiled kernels at that height. Results are the same bits
                            for every choice (block sums are formed over fixed 4-row groups; the sign of a

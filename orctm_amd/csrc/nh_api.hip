@@ -766,11 +766,13 @@ constexpr long long kSmallRowsFew[2] = {256, 512};
 // tiled against streaming: mixed 201x203x13 28 against 30, 203x194x35 47 against 51, 191x259x64 75 against 86,
 // 300x250x60 88 against 97, 379x400x45 96 against 110, 700x600x30 163 against 172 (512x443x25, a width that the tiled
 // ones do not like, 92 against 83); FP64 203x194x35 (776 rows) 68 against 62, 191x259x64 117 against 101, 300x250x60
-// (1250) 151 against 157, 512x443x12 87 against 93, x49 263 against 296, 519x421x5 57 against 59. A context counts as
+// (1250) 151 against 157, 512x443x12 87 against 93, x49 263 against 296; 519x421x5 (3789) 57 against 59,
+// 3183x120x6 (6000) 80 against 88, 1000x1000x6 (16000) 190 against 199. A context counts as
 // one without when most of its rows are: four of 256x256x50, one without, 8.1 ms a solve against 6.8, FP64 13.2
 // against 12.6.
-constexpr int kPlaneLevels[2] = {8, 16};              // FP64, mixed: up to as many levels they stream
-constexpr long long kPlaneRows[2] = {1200, 0};        // and up to as many rows
+bool planes_tiled(int nz, bool fp32, long long rows) {
+  return fp32 ? nz > 16 : nz > 8 ? rows > 1200 : rows > 4000;
+}
 // Columns of one or two levels are outweighed by what the streaming matvec loads once a column, and FP64 columns of few
 // levels in a channel of at most two tiles by the rows that blocks of 4 read twice. us per iteration, tiled against
 // streaming, from the rows at which they lose (below, they are as quick or quicker): one level, 300x420 (2100 rows) 43
@@ -789,7 +791,7 @@ static_assert(kRows32 * 64 <= kSmallColumns, "the columns' sums are kept");
 
 // The kernels that the context's iterations run: blocks of columns (nh_small.h), the streaming ones (nh_stream.h), or
 // the tiled ones, which a forced tile height asks for, and which take what the streaming ones do not hold (more than
-// kStreamLevels levels, arrays past the reach of buffer descriptors) or are no better at (kPlaneLevels, shallow).
+// kStreamLevels levels, arrays past the reach of buffer descriptors) or are no better at (planes_tiled, shallow).
 void ctx_form(Ctx& c, const std::vector<Sys>& systems, const std::vector<int>& forced,
               const std::vector<int>& zw_table) {
   SmallLaunch& l = c.rows;
@@ -807,7 +809,7 @@ void ctx_form(Ctx& c, const std::vector<Sys>& systems, const std::vector<int>& f
   for (int h : forced)
     if (h > 0) return;
   const int prec = c.fp32 ? 1 : 0;
-  const bool tiled = (2 * plane_rows > rows && c.nz > kPlaneLevels[prec] && rows > kPlaneRows[prec]) ||
+  const bool tiled = (2 * plane_rows > rows && planes_tiled(c.nz, c.fp32, rows)) ||
                      shallow(c.nz, c.fp32, rows, narrow_rows);
   const bool stream = c.buf && c.nz <= kStreamLevels && !tiled;
   const bool few = c.nz <= (stream ? kFewLevelsStream : kFewLevels[prec]);

@@ -10,12 +10,12 @@ from orctm_amd.nh import NHBatch, NHSolver, options
 pytestmark = pytest.mark.gpu
 
 # nx, ny, nz, options: rows of 64 columns 256 | 257 and 512 | 513, few and more levels, in reach of the streaming kernels
-# and not; without the table 775, 1200 | 1205 rows; one level 2000 | 2001, two 3100 | 3101, a channel 5000 | 5001
+# and not; without the table 775, 1200 | 1205, 4001 rows; one level 2000 | 2001, two 3100 | 3101, a channel 5000 | 5001
 LINES = [(64, 256, 8, {}), (64, 257, 8, {}), (520, 57, 16, {}), (512, 64, 16, {}), (520, 57, 17, {}),
          (64, 256, 8, {"buffer_addressing": -1}), (64, 257, 8, {"buffer_addressing": -1}),
          (64, 257, 12, {"buffer_addressing": -1}), (64, 257, 13, {"buffer_addressing": -1}), (520, 57, 8, {"buffer_addressing": -1}),
          (260, 155, 16, {"zw_table": -1}), (260, 155, 17, {"zw_table": -1}), (300, 240, 9, {"zw_table": -1}),
-         (300, 241, 9, {"zw_table": -1}), (300, 241, 8, {"zw_table": -1}), (60, 2000, 1, {}), (60, 2001, 1, {}),
+         (300, 241, 9, {"zw_table": -1}), (300, 241, 8, {"zw_table": -1}), (50, 4001, 3, {"zw_table": -1}), (60, 2000, 1, {}), (60, 2001, 1, {}),
          (60, 3100, 2, {}), (60, 3101, 2, {}), (33, 5000, 3, {}), (33, 5001, 3, {}), (33, 5001, 10, {})]
 
 
